@@ -163,14 +163,17 @@ int ensure_mixed(uwshcu_ctx* ctx, size_t ncol) {
     return UWSHCU_OK;
 }
 
-// Columns per launch: as many as the workspace limit allows, a multiple of 64, at
-// least 64 and at most ncol.
+// Columns per launch: the whole chunk where the workspace limit holds it, with the leading
+// dimension rounded up to a wavefront if that fits too; else a multiple of 64 below the
+// limit, at least 64.  A launch takes as long as its slowest column (2-3 ms) however few
+// it holds, so a chunk is never cut for the sake of a round number: rounded down,
+// 12345 columns ran as 12288 and 57 (6.2 ms at 30 levels and 5 constituents, 3.5 ms whole).
 long long batch_columns(const uwshcu_ctx* ctx, int ncol, size_t per_col) {
-    long long nb = (long long)(ctx->ws_limit / per_col);
-    if (nb > ncol) nb = ncol;
-    nb = (nb / 64) * 64;
-    if (nb < 64) nb = 64;
-    return nb;
+    const long long fits = (long long)(ctx->ws_limit / per_col);
+    const long long up = ((long long)ncol + 63) / 64 * 64;
+    if (fits >= up) return up;
+    if (fits >= ncol) return ncol;
+    return fits >= 64 ? fits / 64 * 64 : 64;
 }
 
 struct Chunk {
