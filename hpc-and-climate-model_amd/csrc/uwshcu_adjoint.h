@@ -95,146 +95,44 @@ struct AdGradients {
 // received.  Every adjoint still receives its contributions in decreasing node order,
 // so the result is the same, bit for bit, for every S, and as without a window.
 //
-// The memory operations of a batch are issued together at its end: its far
-// contributions (no-return atomic adds, in step order), then the loads of the adjoints
-// that enter the window and of the next batch's tape nodes (indices clamped into the
-// batch's page), so that one memory latency is paid per batch and no step waits on
-// memory.  (A far contribution can wait to the batch's end: its node enters the window
-// at a later batch's end.)  The page-table entry of a batch is loaded at the end of the
-// batch two before it, so that it has arrived when its nodes are loaded.  Within a
-// step, the node's adjoint and its operands' window entries are
+// A batch's far contributions are added at its end (their nodes enter the window at a later
+// batch's end).  Within a step, the node's adjoint and its operands' window entries are
 // read together and written back unconditionally (an operand outside the window uses
 // the spare entry), so that a step waits for the window once.
-#ifndef UWSHCU_SWEEP_BATCH
-#define UWSHCU_SWEEP_BATCH 16
-#endif
-constexpr int kSweepBatch = UWSHCU_SWEEP_BATCH;
+constexpr int kSweepBatch = 16;   // 16 adjoints are a 128-byte line, 16 nodes three lines
 static_assert(kTapePage % kSweepBatch == 0, "a sweep batch lies within one tape page");
 
-template <class Win>
-UWSHCU_HD inline void ad_reverse(const TapeCtx& t, double* adjv_, const int* nodes, size_t wld, int slot, int mkx,
-                                 int ncnst, size_t ldc, int col, const AdCotangents& cot, const AdGradients& g, Win win,
-                                 int S) {
+// Seed a column's adjoints with the outputs' cotangents.
+UWSHCU_HD inline void ad_seed(UWSHCU_GMEM double* adjv, const int* nodes, size_t wld, int slot, int mkx, int ncnst,
+                              size_t ldc, int col, const AdCotangents& cot) {
     const int KS = mkx + 1;
-    // the header's fields in registers: the sweep's stores could alias the header
-    const TapeCtx th = t;
-    const int n_nodes = th.hot.n;
-    UWSHCU_GMEM double* const adjv = (UWSHCU_GMEM double*)adjv_;
-    auto P = [&](int q) { return adjv + q; };
-    const bool paged = th.pages != nullptr;
-    const UWSHCU_GMEM int* const pages = (const UWSHCU_GMEM int*)th.pages;
-    const UWSHCU_GMEM TapeNode* const pool = paged ? (const UWSHCU_GMEM TapeNode*)th.pool->base : nullptr;
-    const UWSHCU_GMEM TapeNode* const contig = (const UWSHCU_GMEM TapeNode*)th.hot.nodes;   // biased: node q at contig - q
-    // node q of a batch whose page (paged tapes) is pg lives at top(pg) - (q & qmask)
-    const int qmask = paged ? kTapePage - 1 : 0x7fffffff;
-    auto top = [&](int pg) { return paged ? pool + (size_t)pg * kTapePage + (kTapePage - 1) : contig; };
-    auto page_of = [&](int q) { return paged ? pages[q >> kTapePageLog2] : 0; };
     auto node = [&](int f, int k) { return nodes[((size_t)f * KS + k) * wld + slot]; };
     auto row = [&](int k) { return (size_t)(mkx - k) * ldc + col; };
     for (int f = 0; f < ADF_TR; ++f) {
         if (!cot.f[f]) continue;
         for (int k = (f <= ADF_WU ? 0 : 1); k <= mkx; ++k) {
             const int nd = node(f, k);
-            if (nd >= 0) adj_add(P(nd), cot.f[f][row(k)]);
+            if (nd >= 0) adj_add(adjv + nd, cot.f[f][row(k)]);
         }
     }
     if (cot.trten)
         for (int m = 1; m <= ncnst; ++m)
             for (int k = 1; k <= mkx; ++k) {
                 const int nd = node(ADF_TR + m - 1, k);
-                if (nd >= 0) adj_add(P(nd), cot.trten[((size_t)(m - 1) * mkx + (mkx - k)) * ldc + col]);
+                if (nd >= 0) adj_add(adjv + nd, cot.trten[((size_t)(m - 1) * mkx + (mkx - k)) * ldc + col]);
             }
     for (int q = 0; q < ADC_COUNT; ++q) {
         if (!cot.scal[q]) continue;
         const int nd = node(ADF_TR + ncnst + q, 0);
-        if (nd >= 0) adj_add(P(nd), cot.scal[q][col]);
+        if (nd >= 0) adj_add(adjv + nd, cot.scal[q][col]);
     }
-    const int nin = ad_inputs(mkx);
-    const int n = n_nodes;
-    // window entry of node x >= 0 (unsigned: a mask when S is a power of two)
-    auto wslot = [&](int x) { return (int)((unsigned)x % (unsigned)S); };
-    if (S > 0) {
-        constexpr int K = kSweepBatch;
-        double da[K], db[K];
-        int ia[K], ib[K];
-        // the nodes of the batch at q0, clamped into [nin, n - 1] (the same page)
-        auto load_batch = [&](int q0, const UWSHCU_GMEM TapeNode* tb) {
-#pragma unroll
-            for (int u = 0; u < K; ++u) {
-                int q = q0 - u < n - 1 ? q0 - u : n - 1;
-                q = q > nin ? q : nin;
-                const UWSHCU_GMEM TapeNode* p = tb - (q & qmask);
-                da[u] = p->da;
-                db[u] = p->db;
-                ia[u] = p->a;
-                ib[u] = p->b;
-            }
-        };
-        int q0 = (n - 1) | (K - 1);
-        for (int q = n - 1; q >= 0 && q > q0 - S; --q) win(wslot(q)) = adj_load(P(q));
-        if (n > nin) load_batch(q0, top(page_of(n - 1)));
-        // page of the next batch, loaded a batch ahead of its use (clamped to node 0)
-        int pg_next = page_of(q0 - K >= 0 ? q0 - K : 0);
-        for (; q0 >= nin; q0 -= K) {
-            const int lo = q0 - S;     // the window holds the nodes above lo
-            const int lo1 = lo > -1 ? lo : -1;   // an operand a is in the window iff a > lo1
-            int fx[2 * K];             // far contributions of the batch: node (or -1), value
-            double fc[2 * K];
-            // the steps of the batch; kAll: every node of the batch lies in [nin, n - 1]
-            auto steps = [&](auto all) {
-                constexpr bool kAll = decltype(all)::value;
-#pragma unroll
-                for (int u = 0; u < K; ++u) {
-                    // a step outside [nin, n - 1] still runs, on the spare entry, so that
-                    // every path consumes the batch's loads
-                    const int q = q0 - u;
-                    const bool act = kAll || (q >= nin && q < n);
-                    const int a = ia[u], b = ib[u];
-                    const bool nearA = act && a > lo1, nearB = act && b > lo1;
-                    const int sa = nearA ? wslot(a) : S, sb = nearB ? wslot(b) : S;
-                    const double w = win(act ? wslot(q) : S), va = win(sa), vb = win(sb);
-                    const bool live = act && w != 0.0;
-                    const double ca = w * da[u], cb = w * db[u];
-                    fx[2 * u] = live && a >= 0 && !nearA ? a : -1;
-                    fx[2 * u + 1] = live && b >= 0 && !nearB ? b : -1;
-                    fc[2 * u] = ca;
-                    fc[2 * u + 1] = cb;
-                    const double va1 = live && nearA ? va + ca : va;
-                    const double vb0 = nearA && sb == sa ? va1 : vb;    // a == b, both in the window
-                    const double vb1 = live && nearB ? vb0 + cb : vb;
-                    win(sa) = va1;
-                    win(sb) = vb1;
-                }
-            };
-            if (q0 - (K - 1) >= nin && q0 < n) steps(std::true_type{});
-            else steps(std::false_type{});
-            // the batch's far contributions, in step order, then the batch's nodes leave the
-            // window and nodes lo - u enter, into their entries
-#pragma unroll
-            for (int v = 0; v < 2 * K; ++v)
-                if (fx[v] >= 0) adj_add(P(fx[v]), fc[v]);
-            double enter[K];
-#pragma unroll
-            for (int u = 0; u < K; ++u) enter[u] = adj_load(P(lo - u > 0 ? lo - u : 0));
-            const int pg_after = page_of(q0 - 2 * K >= 0 ? q0 - 2 * K : 0);
-            if (q0 - K >= nin) load_batch(q0 - K, top(pg_next));
-            pg_next = pg_after;
-            // written unconditionally (to the spare entry when nothing enters), so that no
-            // load is left pending on some paths into the next batch
-#pragma unroll
-            for (int u = 0; u < K; ++u) win(q0 - u >= nin && lo - u >= 0 ? wslot(q0 - u) : S) = enter[u];
-        }
-    } else {
-        for (int q = n - 1; q >= nin; --q) {
-            const double w = adj_load(P(q));
-            if (w == 0.0) continue;
-            const UWSHCU_GMEM TapeNode& nd = *(top(page_of(q)) - (q & qmask));
-            if (nd.a >= 0) adj_add(P(nd.a), w * nd.da);
-            if (nd.b >= 0) adj_add(P(nd.b), w * nd.db);
-        }
-    }
-    // the inputs' adjoints: the window holds nodes nin - S .. nin - 1, adjv the rest
-    auto A = [&](int q) { return (S > 0 && q >= nin - S) ? win(wslot(q)) : adj_load(P(q)); };
+}
+
+// Write a column's gradients from the inputs' adjoints A(q).
+template <class Adj>
+UWSHCU_HD inline void ad_write_gradients(Adj A, int mkx, size_t ldc, int col, const AdGradients& g) {
+    const int KS = mkx + 1;
+    auto row = [&](int k) { return (size_t)(mkx - k) * ldc + col; };
     for (int k = 1; k <= mkx; ++k) {
         if (g.t0) g.t0[row(k)] = A(ADI_T0 * KS + k);
         if (g.qv0) g.qv0[row(k)] = A(ADI_QV0 * KS + k);
@@ -246,6 +144,88 @@ UWSHCU_HD inline void ad_reverse(const TapeCtx& t, double* adjv_, const int* nod
     if (g.pblh) g.pblh[col] = 0.0;
     if (g.par)
         for (int j = 0; j < 3; ++j) g.par[(size_t)j * ldc + col] = A(ADI_PARAMS * KS + j);
+}
+
+// One step of a windowed sweep: node q, active where act, with operands a, b and partials
+// da, db.  Contributions to nodes above lo1 go to the window; the others are returned in
+// fxa, fxb (node, or -1) and fca, fcb.  A step that is not active runs on the spare entry.
+template <class Win, class Slot>
+UWSHCU_HD inline void ad_step(Win win, Slot wslot, int S, int q, bool act, int lo1, int a, int b, double da, double db,
+                              int& fxa, double& fca, int& fxb, double& fcb) {
+    const bool nearA = act && a > lo1, nearB = act && b > lo1;
+    const int sa = nearA ? wslot(a) : S, sb = nearB ? wslot(b) : S;
+    const double w = win(act ? wslot(q) : S), va = win(sa), vb = win(sb);
+    const bool live = act && w != 0.0;
+    const double ca = w * da, cb = w * db;
+    fxa = live && a >= 0 && !nearA ? a : -1;
+    fxb = live && b >= 0 && !nearB ? b : -1;
+    fca = ca;
+    fcb = cb;
+    const double va1 = live && nearA ? va + ca : va;
+    const double vb0 = nearA && sb == sa ? va1 : vb;    // a == b, both in the window
+    const double vb1 = live && nearB ? vb0 + cb : vb;
+    win(sa) = va1;
+    win(sb) = vb1;
+}
+
+// The sweep of one column by one thread; the GPU's sweep (uwshcu_sweep.hip) takes the same
+// steps in the same order for the columns of a wavefront, whose lanes share the loads.
+template <class Win>
+UWSHCU_HD inline void ad_reverse(const TapeCtx& t, double* adjv_, const int* nodes, size_t wld, int slot, int mkx,
+                                 int ncnst, size_t ldc, int col, const AdCotangents& cot, const AdGradients& g, Win win,
+                                 int S) {
+    // the header's fields in registers: the sweep's stores could alias the header
+    const TapeCtx th = t;
+    UWSHCU_GMEM double* const adjv = (UWSHCU_GMEM double*)adjv_;
+    auto P = [&](int q) { return adjv + q; };
+    const bool paged = th.pages != nullptr;
+    const UWSHCU_GMEM int* const pages = (const UWSHCU_GMEM int*)th.pages;
+    const UWSHCU_GMEM TapeNode* const pool = paged ? (const UWSHCU_GMEM TapeNode*)th.pool->base : nullptr;
+    const UWSHCU_GMEM TapeNode* const contig = (const UWSHCU_GMEM TapeNode*)th.hot.nodes;   // biased: node q at contig - q
+    auto node_at = [&](int q) {
+        return paged ? pool + (size_t)pages[q >> kTapePageLog2] * kTapePage + (kTapePage - 1) - (q & (kTapePage - 1))
+                     : contig - q;
+    };
+    ad_seed(adjv, nodes, wld, slot, mkx, ncnst, ldc, col, cot);
+    const int nin = ad_inputs(mkx);
+    const int n = th.hot.n;
+    // window entry of node x >= 0 (unsigned: a mask when S is a power of two)
+    auto wslot = [&](int x) { return (int)((unsigned)x % (unsigned)S); };
+    if (S > 0) {
+        constexpr int K = kSweepBatch;
+        int q0 = (n - 1) | (K - 1);
+        for (int q = n - 1; q >= 0 && q > q0 - S; --q) win(wslot(q)) = adj_load(P(q));
+        for (; q0 >= nin; q0 -= K) {
+            const int lo = q0 - S;     // the window holds the nodes above lo
+            const int lo1 = lo > -1 ? lo : -1;   // an operand a is in the window iff a > lo1
+            int fx[2 * K];             // far contributions of the batch: node (or -1), value
+            double fc[2 * K];
+            for (int u = 0; u < K; ++u) {
+                const int q = q0 - u;
+                const bool act = q >= nin && q < n;
+                const UWSHCU_GMEM TapeNode* p = node_at(q < nin ? nin : q < n ? q : n - 1);
+                ad_step(win, wslot, S, q, act, lo1, p->a, p->b, p->da, p->db, fx[2 * u], fc[2 * u], fx[2 * u + 1],
+                        fc[2 * u + 1]);
+            }
+            // the batch's far contributions, in step order, then the batch's nodes leave the
+            // window and nodes lo - u enter, into their entries
+            for (int v = 0; v < 2 * K; ++v)
+                if (fx[v] >= 0) adj_add(P(fx[v]), fc[v]);
+            for (int u = 0; u < K; ++u)
+                if (q0 - u >= nin && lo - u >= 0) win(wslot(q0 - u)) = adj_load(P(lo - u));
+        }
+    } else {
+        for (int q = n - 1; q >= nin; --q) {
+            const double w = adj_load(P(q));
+            if (w == 0.0) continue;
+            const UWSHCU_GMEM TapeNode& nd = *node_at(q);
+            if (nd.a >= 0) adj_add(P(nd.a), w * nd.da);
+            if (nd.b >= 0) adj_add(P(nd.b), w * nd.db);
+        }
+    }
+    // the inputs' adjoints: the window holds nodes nin - S .. nin - 1, adjv the rest
+    auto A = [&](int q) { return (S > 0 && q >= nin - S) ? win(wslot(q)) : adj_load(P(q)); };
+    ad_write_gradients(A, mkx, ldc, col, g);
 }
 
 // The window of a sweep without one (S = 0): never read, but the call must bind.

@@ -44,7 +44,10 @@ void adjoint_record_kernel(FwdArgs args, int n, const uwshcu_consts* __restrict_
     col.template run_body<false>();
     col.ad_export(node_out);
     tape.hot = hot;
-    if (tape.overflow == 0) tape.adj = (long long)atomicAdd(&pool->adj_next, (unsigned long long)tape.hot.n);
+    // adjoint entries in whole batches of the sweep, so that each column's start on a cache line
+    if (tape.overflow == 0)
+        tape.adj = (long long)atomicAdd(&pool->adj_next,
+                                        ((unsigned long long)tape.hot.n + kSweepBatch - 1) / kSweepBatch * kSweepBatch);
     else if (tape.overflow == 2) atomicAdd(&pool->retry, 1);
     else record_error(args.err, UWSHCU_ERR_TAPE, args.col0 + j);
     tape.pages = pt;
