@@ -186,25 +186,38 @@ UWSHCU_HD inline double div_rcp(double a, double b, double y) {
 
 // a / b on the GPU by the operations of the hardware's IEEE FP64 division without its
 // range scaling (v_div_scale) and special-value fix-up (v_div_fixup): reciprocal
-// estimate, two Newton steps, quotient, exact remainder and the final fused
-// correction.  When neither operand nor the quotient is near the ends of the
+// estimate, two Newton steps (div_seed), quotient, exact remainder and the final fused
+// correction (div_with).  When neither operand nor the quotient is near the ends of the
 // exponent range (|exponents| below 900, no zero, infinite or NaN divisor) the
 // scaling steps are identities and the fix-up returns its input, so the result is the
-// correctly rounded quotient, the bits of `a / b`; two dependent steps shorter.  Host
-// builds use the operator itself.
-UWSHCU_HD inline double div_fast(double a, double b) {
+// correctly rounded quotient, the bits of `a / b`; two dependent steps shorter.  Several
+// quotients by one divisor share its seed, three operations each.  Host builds use the
+// operator itself.
+UWSHCU_HD inline double div_seed(double b) {
 #if defined(__HIP_DEVICE_COMPILE__)
     double y = __builtin_amdgcn_rcp(b);
     double e = fma(-b, y, 1.0);
     y = fma(y, e, y);
     e = fma(-b, y, 1.0);
-    y = fma(y, e, y);
-    const double q = a * y;
-    return fma(fma(-b, q, a), y, q);
+    return fma(y, e, y);
 #else
+    return b;
+#endif
+}
+UWSHCU_HD inline double div_with(double a, double b, double seed) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double q = a * seed;
+    return fma(fma(-b, q, a), seed, q);
+#else
+    (void)seed;
     return a / b;
 #endif
 }
+UWSHCU_HD inline double div_fast(double a, double b) { return div_with(a, b, div_seed(b)); }
+
+// The upper 32 bits of x: below 0x3ff00000, as an unsigned number, exactly where x is in
+// [0, 1).
+UWSHCU_HD inline unsigned upper_word(double x) { return (unsigned)(__builtin_bit_cast(unsigned long long, x) >> 32); }
 
 }  // namespace uwshcu
 #endif

@@ -14,6 +14,9 @@
 // Every primitive is callable from host code too: the test suite builds the column
 // code for the CPU to check its logic against the oracle before it runs on a GPU.
 #define UWSHCU_HD __host__ __device__
+#ifndef UWSHCU_CONDEN_UNROLL
+#define UWSHCU_CONDEN_UNROLL 5
+#endif
 #ifndef UWSHCU_OUTLINE
 #define UWSHCU_OUTLINE __attribute__((noinline))
 #endif
@@ -135,30 +138,35 @@ struct ThermoT {
 
     // conden_x for D = double: the same operations, each quotient computed so that it
     // has the bits of the plain expression's.
-    //  - Divisions by leff, r and (twice) temps go through correctly rounded
-    //    reciprocals (div_rcp, three dependent operations each).
-    //  - The others, and the reciprocals, use div_fast (no range scaling; every
-    //    operand is a temperature, pressure, latent heat or mixing ratio).
-    //  - The Newton loop keeps the two table entries of the last lookup in registers
-    //    and reads the table again only when the index moves, which after the first
-    //    steps it rarely does.
+    //  - Divisions by leff and r go through correctly rounded reciprocals (div_rcp, three
+    //    operations each), the two by temps share its seed (div_with); the others are
+    //    div_fast (no range scaling; every operand is a temperature, pressure, latent heat
+    //    or mixing ratio).
+    //  - A Newton step has no branch.  A wavefront waits about 45 clocks for a comparison
+    //    that decides a branch, taken or not, and as long at a loop's end, where an FP64
+    //    operation takes 4.6 and the whole step 260: so the table is read in every step (64
+    //    clocks, hidden behind the quotients by temps and leff), five steps make one
+    //    iteration, and the limits of qs, which hold wherever p is above the saturation
+    //    pressure, are checked once after the loop (the steps are taken again with the
+    //    limits if a qs left [0, 1)).  The whole forward: 32768 x 35 x 3 4.54 to 4.37 ms,
+    //    12345 x 30 x 5 3.64 to 3.48 ms, 1 036 800 x 35 x 3 51.4 to 50.9 ms.
     UWSHCU_HD __attribute__((always_inline)) int conden_d(double p, double ex, double thl, double qt, double& th,
                                                          double& qv, double& ql, double& qi,
                                                          SatState* st = nullptr) const {
         const double omeps = 1.0 - c->epsqs;
-        int ic = -1;
-        double tlo = 0.0, thi = 0.0;
-        auto qsat_c = [&](double t, double& es_, double& qs_) {   // qsat_es_qs with the cached entries
+        double tlo, thi;   // table entries of the last lookup
+        auto qsat_free = [&](double t, double& es_, double& qs_) {   // qsat_es_qs without the limits of qs
             const double e = fmax(fmin(t, c->tmax), c->tmin);
-            const int i = (int)(e - c->tmin);
-            if (i != ic) {
-                ic = i;
-                tlo = estbl[i];
-                thi = estbl[i + 1];
-            }
-            const double ai = (double)i;
-            es_ = (c->tmin + ai - e + 1.0) * tlo - (c->tmin + ai - e) * thi;
+            const double d = e - c->tmin;
+            const int i = (int)d;
+            tlo = estbl[i];
+            thi = estbl[i + 1];
+            const double w = c->tmin + trunc(d) - e;
+            es_ = (w + 1.0) * tlo - w * thi;
             qs_ = div_fast(c->epsqs * es_, p - omeps * es_);
+        };
+        auto qsat_c = [&](double t, double& es_, double& qs_) {
+            qsat_free(t, es_, qs_);
             qs_ = fmin(1.0, qs_);
             if (qs_ < 0.0) { qs_ = 1.0; es_ = p; }
         };
@@ -167,7 +175,6 @@ struct ThermoT {
         const double leff = (1.0 - nu) * c->xlv + nu * c->xls;
         double temps = tc, es, qs;
         qsat_c(temps, es, qs);
-        double rvls = qs;
         if (qs >= qt) {
             qv = qt;
             ql = 0.0;
@@ -197,16 +204,28 @@ struct ThermoT {
                 qsat_c(temps, es, qs);
                 if (fabs(temps - tprev) <= 1.e-10 * temps) break;
             }
-            rvls = qs;
         } else {
-            for (int it = 0; it < 10; ++it) {
+            auto step = [&](auto qsat) {
                 tprev = temps;
-                const double rt = div_fast(1.0, temps);
-                const double num = div_rcp((tc - temps) * c->cp, leff, rleff) + qt - rvls;
-                const double d3 = div_rcp(div_rcp(div_rcp(c->ep2 * leff * rvls, c->r, rr), temps, rt), temps, rt);
+                const double seed = div_seed(temps);
+                const double num = div_rcp((tc - temps) * c->cp, leff, rleff) + qt - qs;
+                const double d3 = div_with(div_with(div_rcp(c->ep2 * leff * qs, c->r, rr), temps, seed), temps, seed);
                 temps = temps + div_fast(num, cpl + d3);
-                qsat_c(temps, es, qs);
-                rvls = qs;
+                qsat(temps, es, qs);
+            };
+            const double es0 = es, qs0 = qs;
+            unsigned top = 0;   // the largest upper word of a qs
+#pragma unroll UWSHCU_CONDEN_UNROLL
+            for (int it = 0; it < 10; ++it) {
+                step(qsat_free);
+                top = top > upper_word(qs) ? top : upper_word(qs);
+            }
+            if (__builtin_expect(top >= 0x3ff00000u, 0)) {
+                temps = tc;
+                es = es0;
+                qs = qs0;
+#pragma unroll 1
+                for (int it = 0; it < 10; ++it) step(qsat_c);
             }
         }
         const double qc = fmax(qt - qs, 0.0);
