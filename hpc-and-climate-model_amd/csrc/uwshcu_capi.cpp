@@ -218,9 +218,8 @@ int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pco
     int rc = fixed_ws ? UWSHCU_OK : ensure_ws(ctx, need);
     if (rc) return rc;
     if (recompute && (rc = ensure_mixed(ctx, (size_t)ncol))) return rc;
-    // defer list (nb entries and a counter) and the deferred columns' scalars, for
-    // large launches
-    if (!fixed_ws && nb >= 2 * 1024 * 64 && (size_t)nb + 1 > ctx->defer_cols) {
+    // the split launches' lists and saved scalars
+    if (!fixed_ws && (size_t)nb + 1 > ctx->defer_cols) {
         if (ctx->d_defer) {
             if (!hip_ok(hipDeviceSynchronize())) return UWSHCU_ERR_HIP;
             (void)hipFree(ctx->d_defer);
@@ -296,7 +295,6 @@ int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pco
     a.cush_in = ctx->d_cush_in;
     a.colmap = ctx->d_list;
     a.colcount = ctx->d_count;
-    a.sparse_map = 1;
     a.wld = nb64;
     for (long long c0 = 0; c0 < ncol; c0 += nb64) {
         const int n = (int)((ncol - c0) < nb64 ? (ncol - c0) : nb64);

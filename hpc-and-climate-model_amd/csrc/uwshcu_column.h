@@ -101,57 +101,20 @@ struct FwdArgs {
     // triggered columns run the convection stages, packed densely in a launch of their own
     int defer_at_closure;
     int* defer_mark;         // optional [wld]: mark the deferred column's slot 1 instead of listing it
-    // 1: continue each listed column (colmap) at the closure of its first pass; 2: at its
-    // second convection pass.  Each runs in the workspace slot it had in the deferring
-    // launch (column - slot0), whose set-A environment is intact.
+    // 1: continue each listed column at the closure of its first pass; 2: at its second
+    // convection pass; 4: at the implicit-CIN iteration
     int resume;
+    // those launches run the slots list[0 .. *list_count) of the launch that deferred them
+    // (slot j: column slot0 + j, or colmap[slot0 + j]), whose set-A environment is intact
+    const int* list;
+    const int* list_count;
     int slot0;
-    // 1: colmap lists a few columns of a large range (the mixed mode's FP64 recompute):
-    // run them with the one-wavefront build, unsplit
-    int sparse_map;
     AdArgs ad;               // adjoint kernel only
     // the modified scheme (Column<..., true>): its options, layer omega (caller layout)
     // and the per-column perturbations tpert and qpert
     uwshcu_zw_params zw;
     const double *omega, *tpert, *qpert;
 };
-
-// Level loops whose first level differs between columns (the plume from krel, the
-// penetrative entrainment down from kpen-1) start every lane of a wavefront at the
-// wavefront's extreme first level; a lane runs the loop body only from its own first
-// level on, so its results are those of its own loop.  The lanes then address the same
-// level of the level-major arrays in each iteration, one 64-column row for the
-// wavefront, where lanes at different levels would each read a row of their own.
-// Returns the smallest k among the wavefront's active lanes (the lane's own k on the host).
-UWSHCU_HD inline int wave_min_level(int k) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    int kw = 0;
-    while (__ballot(k <= kw) == 0ull) ++kw;   // ends at this lane's k at the latest
-    return kw;
-#else
-    return k;
-#endif
-}
-UWSHCU_HD inline int wave_max_level(int k) {
-#if defined(__HIP_DEVICE_COMPILE__)
-    int kw = k;
-    while (__ballot(k > kw) != 0ull) ++kw;    // ends at the largest k of the active lanes
-    return kw;
-#else
-    return k;
-#endif
-}
-
-// Parts (bit PART_*) whose level loops align their lanes (wave_min_level).  Alignment
-// makes a wavefront's accesses coalesce, but the lanes idle until their own first level.
-// Measured at 1 036 800 x 35 x 3: aligned, the buoyancy sorting moves 29 GB instead of
-// 49 GB but takes 0.7 ms longer, and the one-wavefront-per-SIMD build loses 10 % at
-// 32768 columns; the stages after the buoyancy sorting, which wait on memory most of the
-// time, gain.  Fastest: those alone (51.4 ms against 52.0 ms unaligned, 52.1 ms aligned
-// in every split part).
-#ifndef UWSHCU_ALIGN_PARTS
-#define UWSHCU_ALIGN_PARTS (1 << PART_REST)
-#endif
 
 // zmh_ramp (mzfunctions_mod.F90:222-248): 0 below x0, 1 above x0 + xint, linear in
 // between; the floor on xint is the single-precision literal 1.e-20 there.
@@ -190,14 +153,20 @@ enum { NRESUME = 57, RS_CONT = 56 };
 // Ints of a split launch's list storage for n columns (launch_column_pipeline).
 UWSHCU_HD inline size_t defer_list_ints(size_t n) { return 3 * n + (n + 255) / 256 + 8; }
 
+// The constituent limiter (S20) moves constituents from this index (1-based) on, but for
+// NUMLIQ and NUMICE, whose tendencies S16 forms from their penetratively entrained values.
+// Updraft values and fluxes of the others enter no output and are not formed.
+enum { kTrLimited = 4 };
+
 // Parts of the column pass that the split pipeline runs as launches of their own.
 // PART_ALL runs whatever FwdArgs::resume asks for; the others fix it at compile time,
 // so that each kernel holds only its own part's live state.
 enum : int {
     PART_ALL = 0,
-    PART_SORT = 1,      // a listed column from its closure through the buoyancy sorting (S11)
+    PART_SORT = 1,      // a listed column from its closure (resume 1) or from the start of its
+                        // second pass (resume 2) through the buoyancy sorting (S11)
     PART_REST = 2,      // the same from the forcedCu filter (S12) through the in-cloud
-                        // diagnostics (S21)
+                        // diagnostics (S21): rest_team (uwshcu_rest.h)
     PART_CLOSURE = 3,   // every column up to the cloud-base closure of its first pass
     PART_CIN2 = 4       // the same, after the level-parallel set-B environment (S22), through
                         // the implicit-CIN iteration's CIN (S1-S7), deferring a second pass
@@ -319,6 +288,11 @@ struct Column {
         if constexpr (kAD) return adout(ADF_TR + m - 1, k);
         else return a.trten[((size_t)(m - 1) * mkx + (mkx - k)) * ldc + i];
     }
+    // constituents (1-based) that S20 moves, and whose entrained values (S13) are read
+    UWSHCU_HD inline bool tr_moved(int m) const { return m >= kTrLimited && m != C.ixnumliq && m != C.ixnumice; }
+    UWSHCU_HD inline bool tr_entrained(int m) const {
+        return m >= kTrLimited || m == C.ixnumliq || m == C.ixnumice;
+    }
     // tunables: j = 0 rpen, 1 rle, 2 rkm
     UWSHCU_HD inline D param(int j) const {
         const double v = j == 0 ? a.par.rpen : j == 1 ? a.par.rle : a.par.rkm;
@@ -413,6 +387,19 @@ struct Column {
         return tv > 0.0;
     }
 
+    // Before a pass.  In a split launch the stages that follow write every level of every
+    // other output and read no working array at a level that they have not written; wu
+    // keeps values of earlier cloud tops, and umf is zero below the inversion.
+    UWSHCU_HD UW_INLINE void start_pass(bool split) const {
+        if (!split) {
+            zero_pass_state();
+            return;
+        }
+        for (int k = 0; k <= mkx; ++k) {
+            out(a.umf, k) = 0.0;
+            out(a.wu, k) = 0.0;
+        }
+    }
     // Zero the column's outputs and the working arrays the reference zeroes before a
     // pass (uwshcu.F90:1333-1408, 1817-1869).
     UWSHCU_HD UW_INLINE void zero_pass_state() const {
@@ -446,27 +433,109 @@ struct Column {
         }
     }
 
-    UWSHCU_HD UW_INLINE void write_exit(int mk) const {
-        // uwshcu.F90:4448-4482; flxprc1/flxsnow1 keep their initial zero (uwshcu.F90:1090-1091)
-        for (int k = 0; k <= mk; ++k) {
-            out(a.umf, k) = 0.0; out(a.wu, k) = 0.0; out(a.slflx, k) = 0.0; out(a.qtflx, k) = 0.0;
-            out(a.flxprc1, k) = 0.0; out(a.flxsnow1, k) = 0.0;
-        }
-        for (int k = 1; k <= mk; ++k) {
-            out(a.qvten, k) = 0.0; out(a.qlten, k) = 0.0; out(a.qiten, k) = 0.0; out(a.sten, k) = 0.0;
-            out(a.uten, k) = 0.0; out(a.vten, k) = 0.0; out(a.qrten, k) = 0.0; out(a.qsten, k) = 0.0;
-            out(a.evapc, k) = 0.0; out(a.cufrc, k) = 0.0; out(a.qcu, k) = 0.0; out(a.qlu, k) = 0.0;
-            out(a.qiu, k) = 0.0; out(a.qc, k) = 0.0;
-            for (int m = 1; m <= ncnst; ++m) trout(m, k) = 0.0;
-        }
-        cout(a.precip) = 0.0; cout(a.snow) = 0.0; cout(a.cush) = -1.0; cout(a.cbmf) = 0.0; cout(a.rliq) = 0.0;
-        cout(a.cnt) = D(mk + 1) - 1.0;        // cnt = 1 flipped: mkx+1-1
-        cout(a.cnb) = D(mk + 1) - D(mk); // cnb = mkx flipped
+    // uwshcu.F90:4448-4482, level k = 0..mkx of a column that exits (layers from 1);
+    // flxprc1/flxsnow1 keep their initial zero (uwshcu.F90:1090-1091)
+    UWSHCU_HD UW_INLINE void zero_outputs_level(int k) const {
+        out(a.umf, k) = 0.0; out(a.wu, k) = 0.0; out(a.slflx, k) = 0.0; out(a.qtflx, k) = 0.0;
+        out(a.flxprc1, k) = 0.0; out(a.flxsnow1, k) = 0.0;
+        if (k < 1) return;
+        out(a.qvten, k) = 0.0; out(a.qlten, k) = 0.0; out(a.qiten, k) = 0.0; out(a.sten, k) = 0.0;
+        out(a.uten, k) = 0.0; out(a.vten, k) = 0.0; out(a.qrten, k) = 0.0; out(a.qsten, k) = 0.0;
+        out(a.evapc, k) = 0.0; out(a.cufrc, k) = 0.0; out(a.qcu, k) = 0.0; out(a.qlu, k) = 0.0;
+        out(a.qiu, k) = 0.0; out(a.qc, k) = 0.0;
+        for (int m = 1; m <= ncnst; ++m) trout(m, k) = 0.0;
     }
+    UWSHCU_HD UW_INLINE void exit_scalars() const {
+        cout(a.precip) = 0.0; cout(a.snow) = 0.0; cout(a.cush) = -1.0; cout(a.cbmf) = 0.0; cout(a.rliq) = 0.0;
+        cout(a.cnt) = D(mkx + 1) - 1.0;        // cnt = 1 flipped: mkx+1-1
+        cout(a.cnb) = D(mkx + 1) - D(mkx); // cnb = mkx flipped
+    }
+    UWSHCU_HD UW_INLINE void write_exit() const {
+        for (int k = 0; k <= mkx; ++k) zero_outputs_level(k);
+        exit_scalars();
+    }
+
+    // The column's diagnostics and branch flag from its saved scalars (rest_team).
+    UWSHCU_HD UW_INLINE void write_diag(int path, int exit_code, int exit_iter, int amb) const {
+        if (a.amb_flag) a.amb_flag[i] = amb;
+        if (!a.diag) return;
+        const size_t L = (size_t)a.ldc;
+        int* d = a.diag + i;
+        d[0 * L] = path == 0 ? exit_code : 0;
+        for (int q = 0; q < 6; ++q) d[(1 + q) * L] = (int)rstate(30 + q);   // kinv klcl klfc krel kbup kpen
+        d[7 * L] = path;
+        for (int q = 0; q < 3; ++q) d[(8 + q) * L] = (int)rstate(36 + q);   // the three limiters
+        d[11 * L] = exit_iter;
+    }
+
+    // S19 positive moisture, FP64 (uwshcu.F90:3995-4001, 5096-5162)
+    UWSHCU_HD UW_INLINE void positive_moisture() const {
+        const double dtd = a.dt;
+        const double qvmin = C.qmin[1], qlmin = C.qmin[2], qimin = C.qmin[3];
+        const double xlvd = C.xlv, xlsd = C.xls;
+        D dqv = 0.0;
+        D carry_qv = 0.0, carry_ten = 0.0;   // adjustments of qv(k-1) and qvten(k-1) from level k
+        bool have_carry = false;
+        for (int k = mkx; k >= 1; --k) {
+            D qvten = out(a.qvten, k), qlten = out(a.qlten, k), qiten = out(a.qiten, k), sten = out(a.sten, k);
+            D qv = in_qv0(k) + qvten * dtd;
+            D ql = in(a.ql0, k) + qlten * dtd;
+            D qi = in(a.qi0, k) + qiten * dtd;
+            if (have_carry) {
+                qv = qv - carry_qv;
+                qvten = qvten - carry_ten;
+            }
+            const D dql = fmax(0.0, 1.0 * qlmin - ql);
+            const D dqi = fmax(0.0, 1.0 * qimin - qi);
+            qlten = qlten + dql / dtd;
+            qiten = qiten + dqi / dtd;
+            qvten = qvten - (dql + dqi) / dtd;
+            sten = sten + xlvd * (dql / dtd) + xlsd * (dqi / dtd);
+            ql = ql + dql;
+            qi = qi + dqi;
+            qv = qv - dql - dqi;
+            dqv = fmax(0.0, 1.0 * qvmin - qv);
+            qvten = qvten + dqv / dtd;
+            qv = qv + dqv;
+            if (k != 1) {
+                const D dpk = in(a.dp0, k), dpkm1 = in(a.dp0, k - 1);
+                carry_qv = dqv * dpk / dpkm1;
+                carry_ten = dqv * dpk / dpkm1 / dtd;
+                have_carry = true;
+            }
+            qv = fmax(qv, qvmin);
+            out(a.qvten, k) = qvten;
+            out(a.qlten, k) = qlten;
+            out(a.qiten, k) = qiten;
+            out(a.sten, k) = sten;
+            E(E_QVSTAR, k) = qv;
+        }
+        if (dqv > 1.e-20) {
+            D sum = 0.0;
+            for (int k = 1; k <= mkx; ++k) {
+                const D qv = E(E_QVSTAR, k);
+                if (qv > 2.0 * qvmin) sum = sum + qv * in(a.dp0, k);
+            }
+            const D aa = dqv * in(a.dp0, 1) / fmax(1.e-20, sum);
+            if (aa < 0.5) {
+                for (int k = 1; k <= mkx; ++k) {
+                    const D qv = E(E_QVSTAR, k);
+                    if (qv > 2.0 * qvmin) {
+                        const D dum = aa * qv;
+                        out(a.qvten, k) = out(a.qvten, k) - dum / dtd;
+                    }
+                }
+            }
+        }
+    }
+
+    // S12-S21 of a listed column, its levels shared by a team of threads (uwshcu_rest.h)
+    template <class Team>
+    UWSHCU_HD __attribute__((always_inline)) void rest_team(Team& tm, bool live, bool final_pass) const;
 
     UWSHCU_HD void run() const { run_body<true>(); }
     template <int PART>
-    UWSHCU_HD void run_part() const { run_body<true, PART>(); }
+    UWSHCU_HD void run_part() const;
     // the column pass itself, expanded into each forward kernel so that each gets its
     // own register allocation (the two builds differ in their register budget).
     // kSplit = false leaves out what only the launches of a split large launch do (stop
@@ -577,19 +646,13 @@ template <class R, class D, bool ZW, bool FAST>
 template <bool kSplit, int PART>
 UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body() const {
     static_assert(PART == PART_ALL || kSplit, "the parts of a split launch need the split build");
+    static_assert(PART != PART_REST, "S12-S21 of a split launch are rest_team");
     // what this launch continues from: 0 the start, 1 the closure of the first pass,
-    // 2 the second convection pass, 3 the forcedCu filter of the first pass, 4 the
-    // implicit-CIN iteration
-    const int resume = PART == PART_SORT ? 1 : PART == PART_REST ? 3 : PART == PART_CLOSURE ? 0
-                     : PART == PART_CIN2 ? 4 : a.resume;
-    if constexpr (PART == PART_REST || PART == PART_CIN2) {
+    // 2 the second convection pass, 4 the implicit-CIN iteration
+    const int resume = PART == PART_CLOSURE ? 0 : PART == PART_CIN2 ? 4 : a.resume;
+    if constexpr (PART == PART_CIN2) {
         if (rstate(RS_CONT) == 0.0) return;      // the column ended in the previous part
     }
-    // level loops with per-column first levels: level-aligned lanes (wave_min_level) in
-    // the parts of UWSHCU_ALIGN_PARTS (bit PART), each lane's own first level elsewhere
-    constexpr bool kAlign = ((UWSHCU_ALIGN_PARTS) >> PART) & 1;
-    auto lvl_lo = [](int k) { return kAlign ? wave_min_level(k) : k; };
-    auto lvl_hi = [](int k) { return kAlign ? wave_max_level(k) : k; };
     // uwshcu.F90:1040-1068 parameters
     const R rmaxfrac = R(0.10), rbuoy = R(1), rdrag = R(1);
     const R PGFc = R(0.7), criqc = R(0.7e-3), frc_rasn = R(1), kevp = R(2.e-6);
@@ -711,7 +774,9 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             if (E(B_THV0BOT, k) < 0.0) { exit_iter = 1; exit_code = EX_CONDEN; goto L333; }
     }
 
-    if (a.env_ready) {
+    if (resume) {
+        // the launch that deferred the column found its environment complete
+    } else if (a.env_ready) {
         for (int k = 1; k <= mkx; ++k)
             if (E(A_THV0BOT, k) < 0.0) { exit_code = EX_CONDEN; goto L333; }
     } else if (!interface_env(A_THL0)) {
@@ -719,21 +784,19 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         goto L333;
     }
 
-    for (int iter = resume ? (kSplit ? (resume == 3 ? 1 : resume == 4 ? 2 : resume) : 2) : 1; iter <= 2; ++iter) {
-        // this pass continues after its buoyancy sorting
-        const bool after_sort = resume == 3 && iter == 1;
+    for (int iter = resume ? (kSplit ? (resume == 4 ? 2 : resume) : 2) : 1; iter <= 2; ++iter) {
         exit_iter = iter;
         const int eb = (iter == 1) ? A_THL0 : B_THL0;        // environment set for S1-S6
         const int e_thl = eb, e_qt = eb + 1, e_ssthl = eb + 2, e_ssqt = eb + 3;
         const int e_thvb = (iter == 1) ? A_THV0BOT : B_THV0BOT, e_thvt = e_thvb + 1;
         const int e_thvlb = (iter == 1) ? A_THVL0BOT : B_THVL0BOT, e_thvlt = e_thvlb + 1;
         const D tscaleh = cush;
-        if (!after_sort) cush = -1.0;   // continued after S11: its cush stands
+        cush = -1.0;
 
-        if (kSplit ? (resume == iter || after_sort) : resume != 0) {
+        if (kSplit ? resume == iter : resume != 0) {
             // a deferred column continues with the scalars it saved: at the second pass
             // those of its implicit-CIN restore, whose convection starts afresh
-            if (!kSplit || iter == 2) zero_pass_state();
+            if (!kSplit || iter == 2) start_pass(PART == PART_SORT);
         } else {
         // ---- S1 kinv (uwshcu.F90:1455-1468) ----
         kinv = 1;
@@ -790,8 +853,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         klfc = mkx;
         if (klcl >= kinv) {
             D thvubot = 0.0, thvutop = 0.0;
-            for (int k = lvl_lo(kinv); k <= mkx - 1; ++k) {
-                if (k < kinv) continue;
+            for (int k = kinv; k <= mkx - 1; ++k) {
                 if (k < klcl) {
                     thvubot = thvlsrc;
                     thvutop = thvlsrc;
@@ -817,8 +879,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             }
         } else {
             cinlcl = 0.0;
-            for (int k = lvl_lo(kinv); k <= mkx - 1; ++k) {
-                if (k < kinv) continue;
+            for (int k = kinv; k <= mkx - 1; ++k) {
                 if (T.conden_x(in(a.ps0, k - 1), E(A_EXNS0, k - 1), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                 const D thvubot = th * (1.0 + C.zvir * qvj - qlj - qij);
                 if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
@@ -870,11 +931,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         {
         R wtw;   // set by the closure, or at the start of the buoyancy sorting
         // a column continued at its first pass (resume 1) resumes at the buoyancy sorting
-        if (kSplit ? !((resume == 1 && iter == 1) || after_sort) : true) {
-        if constexpr (PART == PART_CLOSURE) {
-            zero_pass_state();
-            for (int k = 0; k <= mkx; ++k) { out(a.flxprc1, k) = 0.0; out(a.flxsnow1, k) = 0.0; }
-        }
+        if (kSplit ? !(resume == 1 && iter == 1) : true) {
+        if constexpr (PART == PART_CLOSURE) start_pass(true);
         // ---- S8 release level (uwshcu.F90:2035-2043) ----
         if (klcl < kinv) {
             krel = kinv;
@@ -971,7 +1029,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             W(W_UU, krel - 1) = R(usrc) + uplus;
             W(W_VU, krel - 1) = R(vsrc) + vplus;
         }
-        for (int m = 1; m <= ncnst; ++m) WT(1, m, krel - 1) = R(trin(m, 1));   // trsrc = tr0(1,m)
+        for (int m = kTrLimited; m <= ncnst; ++m) WT(1, m, krel - 1) = R(trin(m, 1));   // trsrc = tr0(1,m)
 
         if (PART == PART_CLOSURE ||
             (PART == PART_ALL && kSplit && iter == 1 && a.defer_at_closure && (a.defer_mark || a.defer_list))) {
@@ -984,7 +1042,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         }   // S8-S10
 
         // ---- S11 buoyancy sorting (uwshcu.F90:2296-2952) ----
-        if (!(kSplit && after_sort)) {   // a column continued after S11 skips it
+        {
         R scaleh = R(tscaleh);
         if (R(tscaleh) < R(0)) scaleh = R(1000);
         for (int iter_scaleh = 1; iter_scaleh <= 3; ++iter_scaleh) {
@@ -1010,8 +1068,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             R c_vu = W(W_VU, krel - 1), c_thvu = W(W_THVU, krel - 1);
             R c_wu = R(out(a.wu, krel - 1)), c_umf = R(out(a.umf, krel - 1));
 
-            for (int k = lvl_lo(krel); k <= mkx - 1; ++k) {
-                if (k < krel) continue;    // level-aligned lanes (wave_min_level)
+            for (int k = krel; k <= mkx - 1; ++k) {
                 const int km1 = k - 1;
                 // Read once for both iter_xc passes: the environment of layer k, which the loop
                 // body does not write, and (issued early) that of layer k+1 for the next level.
@@ -1196,14 +1253,17 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 // Updraft tracers (uwshcu.F90:2592-2614).  Nothing in an iter_xc pass reads
                 // them and each pass overwrites the last, so they are formed once, from the
                 // fer(k) of the pass that ended the loop.
-                if (ferk * dpe < R(1.e-4)) {
-                    for (int m = 1; m <= ncnst; ++m) {
+                if (ncnst < kTrLimited) {
+                } else if (ferk * dpe < R(1.e-4)) {
+                    for (int m = kTrLimited; m <= ncnst; ++m) {
+                        if (!tr_moved(m)) continue;
                         const R tre = tr_mid ? R(trin(m, ktr)) : R(trin(m, ktr)) + WT(0, m, ktr) * pe_tr;
                         WT(1, m, k) = WT(1, m, km1) + (tre + WT(0, m, k) * dpe / R(2) - WT(1, m, km1)) * ferk * dpe;
                     }
                 } else {
                     const R ef = uexp(-ferk * dpe);
-                    for (int m = 1; m <= ncnst; ++m) {
+                    for (int m = kTrLimited; m <= ncnst; ++m) {
+                        if (!tr_moved(m)) continue;
                         const R tre = tr_mid ? R(trin(m, ktr)) : R(trin(m, ktr)) + WT(0, m, ktr) * pe_tr;
                         const R sst = WT(0, m, k);
                         WT(1, m, k) = (tre + sst / ferk - sst * dpe / R(2)) -
@@ -1314,11 +1374,12 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         }
         if constexpr (PART == PART_SORT) {
             // the rest of the pass runs in the next launch: save what S11 set (the other
-            // saved scalars still hold the closure's values) and stop
+            // saved scalars still hold the closure's values, but for a second pass, whose
+            // closure ran here)
             resume_io([&](int f, auto& x) {
-                const bool set_here = f == 0 || (f >= 18 && f <= 29) || f == 34 || f == 35 || f == 36 ||
-                                      f == 37 || f == 39;
-                if (!set_here) return;
+                const bool set_here = f == 0 || (f >= 18 && f <= 20) || (f >= 34 && f <= 37) || f == 39;
+                const bool closure = iter == 2 && ((f >= 13 && f <= 17) || f == 33);
+                if (!set_here && !closure) return;
                 if constexpr (std::is_integral<std::remove_reference_t<decltype(x)>>::value) rstate(f) = (double)x;
                 else rstate(f) = (double)val(x);
             });
@@ -1329,23 +1390,15 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
 
         // ---- S12 forcedCu filter (uwshcu.F90:2964-2992) ----
         if (kbup == krel) { exit_code = EX_CUFILTER; goto L333; }
-        for (int k = lvl_lo(kpen); k <= mkx; ++k) {
-            if (k < kpen) continue;
+        for (int k = kpen; k <= mkx; ++k) {
             out(a.umf, k) = 0.0; W(W_EMF, k) = R(0); W(W_UFRC, k) = R(0);
             if (k == kpen) continue;
             W(W_DWTEN, k) = R(0); W(W_DITEN, k) = R(0); W(W_FER, k) = R(0); W(W_FDR, k) = R(0);
         }
 
         // ---- S13 penetrative entrainment (uwshcu.F90:3055-3183) ----
-        for (int k = 0; k <= mkx; ++k) {
-            W(W_THLUE, k) = W(W_THLU, k);
-            W(W_QTUE, k) = W(W_QTU, k);
-            W(W_UUE, k) = W(W_UU, k);
-            W(W_VUE, k) = W(W_VU, k);
-            for (int m = 1; m <= ncnst; ++m) WT(2, m, k) = WT(1, m, k);
-        }
-        for (int k = lvl_hi(kpen - 1); k >= kbup; --k) {
-            if (k > kpen - 1) continue;
+        // (thlue and its like are read from kbup to kpen - 1 only, where this loop sets them)
+        for (int k = kpen - 1; k >= kbup; --k) {
             const R rhos0j = R(in(a.ps0, k)) / (r * R(0.5) * (Er(A_THV0BOT, k + 1) + Er(A_THV0TOP, k)) * Er(A_EXNS0, k));
             const R umfk = R(out(a.umf, k));
             if (k == kpen - 1) {
@@ -1359,7 +1412,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 W(W_QTUE, k) = Er(A_QT0, kpen) + Er(A_SSQT0, kpen) * dpk;
                 W(W_UUE, k) = R(in(a.u0, kpen)) + Er(A_SSU0, kpen) * dpk;
                 W(W_VUE, k) = R(in(a.v0, kpen)) + Er(A_SSV0, kpen) * dpk;
-                for (int m = 1; m <= ncnst; ++m) WT(2, m, k) = R(trin(m, kpen)) + WT(0, m, kpen) * dpk;
+                for (int m = 1; m <= ncnst; ++m)
+                    if (tr_entrained(m)) WT(2, m, k) = R(trin(m, kpen)) + WT(0, m, kpen) * dpk;
             } else {
                 const R emf1 = W(W_EMF, k + 1);
                 const R x = emf1 - umfk * R(in(a.dp0, k + 1)) * W(W_REI, k + 1) * rpen;
@@ -1375,13 +1429,15 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                     W(W_UUE, k) = (W(W_UUE, k + 1) * emf1 + R(in(a.u0, k + 1)) * (emfk - emf1)) / emfk;
                     W(W_VUE, k) = (W(W_VUE, k + 1) * emf1 + R(in(a.v0, k + 1)) * (emfk - emf1)) / emfk;
                     for (int m = 1; m <= ncnst; ++m)
-                        WT(2, m, k) = (WT(2, m, k + 1) * emf1 + R(trin(m, k + 1)) * (emfk - emf1)) / emfk;
+                        if (tr_entrained(m))
+                            WT(2, m, k) = (WT(2, m, k + 1) * emf1 + R(trin(m, k + 1)) * (emfk - emf1)) / emfk;
                 } else {
                     W(W_THLUE, k) = Er(A_THL0, k + 1);
                     W(W_QTUE, k) = Er(A_QT0, k + 1);
                     W(W_UUE, k) = R(in(a.u0, k + 1));
                     W(W_VUE, k) = R(in(a.v0, k + 1));
-                    for (int m = 1; m <= ncnst; ++m) WT(2, m, k) = R(trin(m, k + 1));
+                    for (int m = 1; m <= ncnst; ++m)
+                    if (tr_entrained(m)) WT(2, m, k) = R(trin(m, k + 1));
                 }
             }
         }
@@ -1422,7 +1478,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             fluxbelowinv(R(vsrc), R(in(a.v0, kinv)), R(in(a.v0, kinv + 1)) + Er(A_SSV0, kinv + 1) * dtop,
                          R(in(a.v0, kinv - 1)) + Er(A_SSV0, kinv - 1) * dbot,
                          [&](int k, R x) { W(W_VFLX, k) = x; });
-            for (int m = 1; m <= ncnst; ++m) {
+            for (int m = kTrLimited; m <= ncnst; ++m) {
+                if (!tr_moved(m)) continue;
                 fluxbelowinv(R(trin(m, 1)), R(trin(m, kinv)), R(trin(m, kinv + 1)) + WT(0, m, kinv + 1) * dtop,
                              R(trin(m, kinv - 1)) + WT(0, m, kinv - 1) * dbot,
                              [&](int k, R x) { WT(3, m, k) = x; });
@@ -1430,8 +1487,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         }
         {
             R uplus = R(0), vplus = R(0);
-            for (int k = lvl_lo(kinv); k <= krel - 1; ++k) {
-                if (k < kinv) continue;
+            for (int k = kinv; k <= krel - 1; ++k) {
                 const int kp1 = k + 1;
                 const R d = R(in(a.ps0, k) - in(a.p0, kp1));
                 out(a.qtflx, k) = D(cbmf * (R(qtsrc) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
@@ -1440,12 +1496,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 vplus = vplus + PGFc * Er(A_SSV0, k) * R(in(a.ps0, k) - in(a.ps0, k - 1));
                 W(W_UFLX, k) = cbmf * (R(usrc) + uplus - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
                 W(W_VFLX, k) = cbmf * (R(vsrc) + vplus - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
-                for (int m = 1; m <= ncnst; ++m)
-                    WT(3, m, k) = cbmf * (R(trin(m, 1)) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
+                for (int m = kTrLimited; m <= ncnst; ++m)
+                    if (tr_moved(m)) WT(3, m, k) = cbmf * (R(trin(m, 1)) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
             }
         }
-        for (int k = lvl_lo(krel); k <= kbup - 1; ++k) {
-            if (k < krel) continue;
+        for (int k = krel; k <= kbup - 1; ++k) {
             const int kp1 = k + 1;
             const R d = R(in(a.ps0, k) - in(a.p0, kp1));
             const R umfk = R(out(a.umf, k));
@@ -1453,19 +1508,18 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             out(a.qtflx, k) = D(umfk * (W(W_QTU, k) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
             W(W_UFLX, k) = umfk * (W(W_UU, k) - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
             W(W_VFLX, k) = umfk * (W(W_VU, k) - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
-            for (int m = 1; m <= ncnst; ++m)
-                WT(3, m, k) = umfk * (WT(1, m, k) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
+            for (int m = kTrLimited; m <= ncnst; ++m)
+                if (tr_moved(m)) WT(3, m, k) = umfk * (WT(1, m, k) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
         }
-        for (int k = lvl_lo(kbup); k <= kpen - 1; ++k) {
-            if (k < kbup) continue;
+        for (int k = kbup; k <= kpen - 1; ++k) {
             const R d = R(in(a.ps0, k) - in(a.p0, k));
             const R emfk = W(W_EMF, k);
             out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * emfk * (W(W_THLUE, k) - (Er(A_THL0, k) + Er(A_SSTHL0, k) * d)));
             out(a.qtflx, k) = D(emfk * (W(W_QTUE, k) - (Er(A_QT0, k) + Er(A_SSQT0, k) * d)));
             W(W_UFLX, k) = emfk * (W(W_UUE, k) - (R(in(a.u0, k)) + Er(A_SSU0, k) * d));
             W(W_VFLX, k) = emfk * (W(W_VUE, k) - (R(in(a.v0, k)) + Er(A_SSV0, k) * d));
-            for (int m = 1; m <= ncnst; ++m)
-                WT(3, m, k) = emfk * (WT(2, m, k) - (R(trin(m, k)) + WT(0, m, k) * d));
+            for (int m = kTrLimited; m <= ncnst; ++m)
+                if (tr_moved(m)) WT(3, m, k) = emfk * (WT(2, m, k) - (R(trin(m, k)) + WT(0, m, k) * d));
         }
 
         // ---- S15 subsidence condensate sinks (uwshcu.F90:3416-3476) ----
@@ -1706,69 +1760,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             out(a.sten, k) = D(R(out(a.sten, k)) - (xls - xlv) * W(W_QCI, k));
         }
 
-        // ---- S19 positive moisture, FP64 (uwshcu.F90:3995-4001, 5096-5162) ----
-        {
-            const double qvmin = C.qmin[1], qlmin = C.qmin[2], qimin = C.qmin[3];
-            const double xlvd = C.xlv, xlsd = C.xls;
-            D dqv = 0.0;
-            D carry_qv = 0.0, carry_ten = 0.0;   // adjustments of qv(k-1) and qvten(k-1) from level k
-            bool have_carry = false;
-            for (int k = mkx; k >= 1; --k) {
-                D qvten = out(a.qvten, k), qlten = out(a.qlten, k), qiten = out(a.qiten, k), sten = out(a.sten, k);
-                D qv = in_qv0(k) + qvten * dtd;
-                D ql = in(a.ql0, k) + qlten * dtd;
-                D qi = in(a.qi0, k) + qiten * dtd;
-                if (have_carry) {
-                    qv = qv - carry_qv;
-                    qvten = qvten - carry_ten;
-                }
-                const D dql = fmax(0.0, 1.0 * qlmin - ql);
-                const D dqi = fmax(0.0, 1.0 * qimin - qi);
-                qlten = qlten + dql / dtd;
-                qiten = qiten + dqi / dtd;
-                qvten = qvten - (dql + dqi) / dtd;
-                sten = sten + xlvd * (dql / dtd) + xlsd * (dqi / dtd);
-                ql = ql + dql;
-                qi = qi + dqi;
-                qv = qv - dql - dqi;
-                dqv = fmax(0.0, 1.0 * qvmin - qv);
-                qvten = qvten + dqv / dtd;
-                qv = qv + dqv;
-                if (k != 1) {
-                    const D dpk = in(a.dp0, k), dpkm1 = in(a.dp0, k - 1);
-                    carry_qv = dqv * dpk / dpkm1;
-                    carry_ten = dqv * dpk / dpkm1 / dtd;
-                    have_carry = true;
-                }
-                qv = fmax(qv, qvmin);
-                out(a.qvten, k) = qvten;
-                out(a.qlten, k) = qlten;
-                out(a.qiten, k) = qiten;
-                out(a.sten, k) = sten;
-                E(E_QVSTAR, k) = qv;
-            }
-            if (dqv > 1.e-20) {
-                D sum = 0.0;
-                for (int k = 1; k <= mkx; ++k) {
-                    const D qv = E(E_QVSTAR, k);
-                    if (qv > 2.0 * qvmin) sum = sum + qv * in(a.dp0, k);
-                }
-                const D aa = dqv * in(a.dp0, 1) / fmax(1.e-20, sum);
-                if (aa < 0.5) {
-                    for (int k = 1; k <= mkx; ++k) {
-                        const D qv = E(E_QVSTAR, k);
-                        if (qv > 2.0 * qvmin) {
-                            const D dum = aa * qv;
-                            out(a.qvten, k) = out(a.qvten, k) - dum / dtd;
-                        }
-                    }
-                }
-            }
-        }
+        positive_moisture();   // S19
 
         // ---- S20 constituent limiter (uwshcu.F90:4007-4076) ----
         for (int m = 4; m <= ncnst; ++m) {
-            if (m == ixl || m == ixi) continue;
+            if (!tr_moved(m)) continue;
             const R trmin = R(C.qmin[m]);
             const bool wet = C.wet[m] != 0;
             auto pdelx = [&](int k) -> R { return wet ? R(in(a.dp0, k)) : R(in(a.dpdry0, k)); };
@@ -1795,9 +1791,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         {
             // the tendency stage adjusted the same updraft states: reuse its condensate
             R qcubelow = qlr_base + qir_base, qlubelow = qlr_base, qiubelow = qir_base;
-            for (int k = lvl_lo(krel); k <= kpen; ++k) {
-                if (k < krel) continue;
-                const R qlr = W(W_QLR, k), qir = W(W_QIR, k);
+            for (int k = krel; k <= kpen; ++k) {
+                    const R qlr = W(W_QLR, k), qir = W(W_QIR, k);
                 R qcuk = R(0.5) * (qcubelow + qlr + qir);
                 R qluk = R(0.5) * (qlubelow + qlr);
                 R qiuk = R(0.5) * (qiubelow + qir);
@@ -1844,18 +1839,6 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         cout(a.cnt) = D(mkx + 1 - kpen);
         cout(a.cnb) = D(mkx + 1 - (krel - 1));
 
-        if constexpr (PART == PART_REST) {
-            // S22 runs level-parallel (setup_level_b1/b2) and the implicit-CIN iteration in
-            // a launch of its own: save what S12-S21 set and stop
-            resume_io([&](int f, auto& x) {
-                if (!((f >= 26 && f <= 29) || f == 38 || f == 39)) return;
-                if constexpr (std::is_integral<std::remove_reference_t<decltype(x)>>::value) rstate(f) = (double)x;
-                else rstate(f) = (double)val(x);
-            });
-            rstate(RS_CONT) = 1.0;
-            return;
-        }
-
         // ---- S22 provisional state and environment set B (uwshcu.F90:4169-4329) ----
         if (iter == 1) {
             cush_s = cush;
@@ -1881,9 +1864,9 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
     goto Ldone;
 
 L333:
-    write_exit(mkx);
+    write_exit();
     path = 0;
-    if constexpr (PART == PART_SORT || PART == PART_REST) rstate(RS_CONT) = 0.0;
+    if constexpr (PART == PART_SORT) rstate(RS_CONT) = 0.0;
 
 Ldone:
     if (a.amb_flag) a.amb_flag[i] = amb;
@@ -1893,6 +1876,23 @@ Ldone:
         d[0 * L] = (path == 0) ? exit_code : 0;
         d[1 * L] = kinv; d[2 * L] = klcl; d[3 * L] = klfc; d[4 * L] = krel; d[5 * L] = kbup; d[6 * L] = kpen;
         d[7 * L] = path; d[8 * L] = limit_ufrc; d[9 * L] = limit_ppen; d[10 * L] = limit_emf; d[11 * L] = exit_iter;
+    }
+}
+
+}  // namespace uwshcu
+
+#include "uwshcu_rest.h"
+
+namespace uwshcu {
+
+template <class R, class D, bool ZW, bool FAST>
+template <int PART>
+UWSHCU_HD void Column<R, D, ZW, FAST>::run_part() const {
+    if constexpr (PART == PART_REST) {
+        SerialTeam one;
+        rest_team(one, true, false);
+    } else {
+        run_body<true, PART>();
     }
 }
 

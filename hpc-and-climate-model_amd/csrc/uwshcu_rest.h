@@ -1,0 +1,640 @@
+// uwshcu_rest.h -- the stages after the buoyancy sorting (S12-S21), level-parallel.
+//
+// A column's fluxes, subsidence sinks, tendencies and diagnostics at one level depend on
+// other levels only through a few recurrences: the penetrative entrainment (S13, down from
+// the cloud top over one to three levels), the precipitation evaporation (S17, down the
+// column), the moisture borrowed from the layer below (S19, only where a layer runs dry)
+// and the constituent limiter (S20, one constituent at a time).  Everything else runs one
+// thread per column and level.
+//
+// What bounds it: memory.  One thread per column waited 82 % of its time on these stages,
+// on rows that lie a whole level apart, at two wavefronts per SIMD (14.8 ms of 51.4 at
+// 1 036 800 x 35 x 3, most of a small launch's second half).  Here a workgroup takes 64
+// columns of the list and its wavefronts the levels in turn, so a column has as many
+// accesses in flight as there are wavefronts, and a wavefront's accesses stay one
+// 64-column row per array and level: 9.9 ms there, 35 GB moved; 0.4 ms at 32768 columns.
+//
+// The same code runs on the host with a team of one (every stage over all levels in
+// turn).  Each value is computed by the sequential stages' operations in their order, so
+// the results are those of Column::run_body's S12-S21 bit for bit.
+#ifndef UWSHCU_REST_H
+#define UWSHCU_REST_H
+
+#include "uwshcu_column.h"
+
+namespace uwshcu {
+
+// A team of one thread: takes every level.
+struct SerialTeam {
+    int fail_key = 0x7fffffff, borrow = 0;
+    static constexpr int rank = 0, size = 1;
+    UWSHCU_HD void sync() {}
+    UWSHCU_HD void fail(int key) { fail_key = key < fail_key ? key : fail_key; }
+    UWSHCU_HD int failed() const { return fail_key; }
+    UWSHCU_HD void borrows() { borrow = 1; }
+    UWSHCU_HD bool borrowed() const { return borrow != 0; }
+};
+
+// live: this thread's column takes part (every thread of a team calls this, for the
+// team's synchronisations).  final_pass: the second convection pass; else the first.
+template <class R, class D, bool ZW, bool FAST>
+template <class Team>
+UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(Team& tm, bool live, bool final_pass) const {
+    const R rmaxfrac = R(0.10);
+    const R PGFc = R(0.7), criqc = R(0.7e-3), frc_rasn = R(1), kevp = R(2.e-6);
+    const R xlv = R(C.xlv), xls = R(C.xls), cp = R(C.cp), r = R(C.r), g = R(C.g);
+    const R rpen = R(param(0));
+    const R dt = R(a.dt);
+    const double dtd = a.dt;
+    const int ixl = C.ixnumliq, ixi = C.ixnumice;
+    const bool has_nl = ixl >= 1 && ixl <= ncnst, has_ni = ixi >= 1 && ixi <= ncnst;
+    auto trz = [&](int m, int k) -> R { return (m >= 1 && m <= ncnst) ? R(trin(m, k)) : R(0); };
+    constexpr bool kFp32 = sizeof(R) == sizeof(float);
+    constexpr double kGuard = kFp32 ? 1.e-5 : 1.e-8;
+    int amb = 0;
+    auto near = [&](auto dist, auto scale) {   // the branch guard of run_body
+        if constexpr (kFp32 || FAST) {
+            if (fabs(dist) <= kGuard * fabs(scale)) amb = 1;
+        }
+    };
+    const int w = tm.rank, nw = tm.size;
+    const bool lead = w == 0;
+
+    int kinv = 0, krel = 0, kbup = 0, kpen = -1;
+    R prel = 0, cbmf = 0, ufrclcl = 0, ppen = 0, thlu_top = 0, qtu_top = 0;
+    D qtsrc = 0, thlsrc = 0, usrc = 0, vsrc = 0;
+    int code = EX_NONE;
+    live = live && rstate(RS_CONT) != 0.0;
+    if (live) {
+        qtsrc = rstate(7); thlsrc = rstate(9); usrc = rstate(10); vsrc = rstate(11);
+        prel = R(rstate(13)); cbmf = R(rstate(15)); ufrclcl = R(rstate(17)); ppen = R(rstate(18));
+        thlu_top = R(rstate(19)); qtu_top = R(rstate(20));
+        kinv = (int)rstate(30); krel = (int)rstate(33); kbup = (int)rstate(34); kpen = (int)rstate(35);
+        amb = (int)rstate(39);
+        if (kbup == krel) code = EX_CUFILTER;   // ---- S12 forcedCu filter (uwshcu.F90:2964-2992) ----
+    }
+    bool run = live && code == EX_NONE;
+    int limit_emf = 0;
+
+    if (run) {
+        for (int k = w; k <= mkx; k += nw)
+            if (k >= kpen) out(a.umf, k) = 0.0;
+
+        // ---- S13 penetrative entrainment (uwshcu.F90:3055-3183) ----
+        if (lead) {
+            limit_emf = (int)rstate(38);
+            R emf1 = 0, thlue1 = 0, qtue1 = 0, uue1 = 0, vue1 = 0;   // level k + 1
+            for (int k = kpen - 1; k >= kbup; --k) {
+                const R rhos0j = R(in(a.ps0, k)) / (r * R(0.5) * (Er(A_THV0BOT, k + 1) + Er(A_THV0TOP, k)) * Er(A_EXNS0, k));
+                const R umfk = R(out(a.umf, k));
+                R emfk, thluek, qtuek, uuek, vuek;
+                if (k == kpen - 1) {
+                    const R x = umfk * ppen * W(W_REI, kpen) * rpen;
+                    const R lim2 = R(-0.9) * R(in(a.dp0, kpen)) / g / dt;
+                    if (x < R(-0.1) * rhos0j) limit_emf = 1;
+                    if (x < lim2) limit_emf = 1;
+                    emfk = fmax(fmax(x, R(-0.1) * rhos0j), lim2);
+                    const R dpk = R(in(a.ps0, k) - in(a.p0, kpen));
+                    thluek = Er(A_THL0, kpen) + Er(A_SSTHL0, kpen) * dpk;
+                    qtuek = Er(A_QT0, kpen) + Er(A_SSQT0, kpen) * dpk;
+                    uuek = R(in(a.u0, kpen)) + Er(A_SSU0, kpen) * dpk;
+                    vuek = R(in(a.v0, kpen)) + Er(A_SSV0, kpen) * dpk;
+                    for (int m = 1; m <= ncnst; ++m)
+                            if (tr_entrained(m)) WT(2, m, k) = R(trin(m, kpen)) + WT(0, m, kpen) * dpk;
+                } else {
+                    const R x = emf1 - umfk * R(in(a.dp0, k + 1)) * W(W_REI, k + 1) * rpen;
+                    const R lim2 = R(-0.9) * R(in(a.dp0, k + 1)) / g / dt;
+                    if (x < R(-0.1) * rhos0j) limit_emf = 1;
+                    if (x < lim2) limit_emf = 1;
+                    emfk = fmax(fmax(x, R(-0.1) * rhos0j), lim2);
+                    near(fabs(emfk) - fabs(emf1), fabs(emf1));
+                    if (fabs(emfk) > fabs(emf1)) {
+                        thluek = (thlue1 * emf1 + Er(A_THL0, k + 1) * (emfk - emf1)) / emfk;
+                        qtuek = (qtue1 * emf1 + Er(A_QT0, k + 1) * (emfk - emf1)) / emfk;
+                        uuek = (uue1 * emf1 + R(in(a.u0, k + 1)) * (emfk - emf1)) / emfk;
+                        vuek = (vue1 * emf1 + R(in(a.v0, k + 1)) * (emfk - emf1)) / emfk;
+                        for (int m = 1; m <= ncnst; ++m)
+                                if (tr_entrained(m))
+                                    WT(2, m, k) = (WT(2, m, k + 1) * emf1 + R(trin(m, k + 1)) * (emfk - emf1)) / emfk;
+                    } else {
+                        thluek = Er(A_THL0, k + 1);
+                        qtuek = Er(A_QT0, k + 1);
+                        uuek = R(in(a.u0, k + 1));
+                        vuek = R(in(a.v0, k + 1));
+                        for (int m = 1; m <= ncnst; ++m)
+                            if (tr_entrained(m)) WT(2, m, k) = R(trin(m, k + 1));
+                    }
+                }
+                W(W_EMF, k) = emfk;
+                W(W_THLUE, k) = thluek;
+                W(W_QTUE, k) = qtuek;
+                W(W_UUE, k) = uuek;
+                W(W_VUE, k) = vuek;
+                emf1 = emfk; thlue1 = thluek; qtue1 = qtuek; uue1 = uuek; vue1 = vuek;
+            }
+            rstate(38) = (double)limit_emf;
+        }
+
+        // ---- S14 fluxes below the cloud top (uwshcu.F90:3255-3401) ----
+        {
+            // fluxbelowinv (uwshcu.F90:5030-5094) for one scalar; writes xflx(0..kinv-1) via put
+            auto fluxbelowinv = [&](R xsrc, R xmean, R xtopin, R xbotin, auto put) {
+                const R dp = R(in(a.ps0, kinv - 1) - in(a.ps0, kinv));
+                R xbot, xtop;
+                if (fabs(xbotin - xtopin) <= R(1.e-13)) { xbot = xbotin - R(1.e-13); xtop = xtopin + R(1.e-13); }
+                else { xbot = xbotin; xtop = xtopin; }
+                const R xtop_ori = xtop, xbot_ori = xbot;
+                const R rcbmf = (cbmf * g * dt) / dp;
+                R rpeff = (xmean - xtop) / (xbot - xtop);
+                rpeff = fmin(fmax(R(0), rpeff), R(1));
+                if (rpeff == R(0) || rpeff == R(1)) { xbot = xmean; xtop = xmean; }
+                const R rr = rpeff / rcbmf;
+                const R pinv = R(in(a.ps0, kinv - 1)) - rpeff * dp;
+                const R ps00 = R(in(a.ps0, 0));
+                for (int k = w; k <= kinv - 1; k += nw) {
+                    R x = cbmf * (xsrc - xbot) * (ps00 - R(in(a.ps0, k))) / (ps00 - pinv);
+                    if (k == kinv - 1 && rr <= R(1)) x = x - (R(1) - rr) * cbmf * (xtop_ori - xbot_ori);
+                    put(k, x);
+                }
+            };
+            if (w <= kinv - 1) {
+                const R dtop = R(in(a.ps0, kinv) - in(a.p0, kinv + 1));
+                const R dbot = R(in(a.ps0, kinv - 1) - in(a.p0, kinv - 1));
+                fluxbelowinv(R(qtsrc), Er(A_QT0, kinv), Er(A_QT0, kinv + 1) + Er(A_SSQT0, kinv + 1) * dtop,
+                             Er(A_QT0, kinv - 1) + Er(A_SSQT0, kinv - 1) * dbot,
+                             [&](int k, R x) { out(a.qtflx, k) = D(x); });
+                fluxbelowinv(R(thlsrc), Er(A_THL0, kinv), Er(A_THL0, kinv + 1) + Er(A_SSTHL0, kinv + 1) * dtop,
+                             Er(A_THL0, kinv - 1) + Er(A_SSTHL0, kinv - 1) * dbot,
+                             [&](int k, R x) { out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * x); });
+                fluxbelowinv(R(usrc), R(in(a.u0, kinv)), R(in(a.u0, kinv + 1)) + Er(A_SSU0, kinv + 1) * dtop,
+                             R(in(a.u0, kinv - 1)) + Er(A_SSU0, kinv - 1) * dbot,
+                             [&](int k, R x) { W(W_UFLX, k) = x; });
+                fluxbelowinv(R(vsrc), R(in(a.v0, kinv)), R(in(a.v0, kinv + 1)) + Er(A_SSV0, kinv + 1) * dtop,
+                             R(in(a.v0, kinv - 1)) + Er(A_SSV0, kinv - 1) * dbot,
+                             [&](int k, R x) { W(W_VFLX, k) = x; });
+                for (int m = kTrLimited; m <= ncnst; ++m) {
+                    if (!tr_moved(m)) continue;
+                    fluxbelowinv(R(trin(m, 1)), R(trin(m, kinv)), R(trin(m, kinv + 1)) + WT(0, m, kinv + 1) * dtop,
+                                 R(trin(m, kinv - 1)) + WT(0, m, kinv - 1) * dbot,
+                                 [&](int k, R x) { WT(3, m, k) = x; });
+                }
+            }
+        }
+        for (int k = w; k <= kbup - 1; k += nw) {
+            if (k < kinv) continue;
+            const int kp1 = k + 1;
+            const R d = R(in(a.ps0, k) - in(a.p0, kp1));
+            if (k <= krel - 1) {
+                R uplus = R(0), vplus = R(0);
+                for (int q = kinv; q <= k; ++q) {
+                    uplus = uplus + PGFc * Er(A_SSU0, q) * R(in(a.ps0, q) - in(a.ps0, q - 1));
+                    vplus = vplus + PGFc * Er(A_SSV0, q) * R(in(a.ps0, q) - in(a.ps0, q - 1));
+                }
+                out(a.qtflx, k) = D(cbmf * (R(qtsrc) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
+                out(a.slflx, k) = D(cbmf * (R(thlsrc) - (Er(A_THL0, kp1) + Er(A_SSTHL0, kp1) * d)) * cp * Er(A_EXNS0, k));
+                W(W_UFLX, k) = cbmf * (R(usrc) + uplus - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
+                W(W_VFLX, k) = cbmf * (R(vsrc) + vplus - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
+                for (int m = kTrLimited; m <= ncnst; ++m)
+                    if (tr_moved(m)) WT(3, m, k) = cbmf * (R(trin(m, 1)) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
+            } else {
+                const R umfk = R(out(a.umf, k));
+                out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * umfk * (W(W_THLU, k) - (Er(A_THL0, kp1) + Er(A_SSTHL0, kp1) * d)));
+                out(a.qtflx, k) = D(umfk * (W(W_QTU, k) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
+                W(W_UFLX, k) = umfk * (W(W_UU, k) - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
+                W(W_VFLX, k) = umfk * (W(W_VU, k) - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
+                for (int m = kTrLimited; m <= ncnst; ++m)
+                    if (tr_moved(m)) WT(3, m, k) = umfk * (WT(1, m, k) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
+            }
+        }
+        // updraft condensate at the layer tops, and at the release level (kept at krel - 1),
+        // which the tendencies and the in-cloud diagnostics share
+        for (int k = w; k <= kpen; k += nw) {
+            if (k < krel) continue;
+            D th, qvj, qlj, qij;
+            int bad;
+            if (k == krel) {
+                if (T.conden(prel, W(W_THLU, krel - 1), W(W_QTU, krel - 1), th, qvj, qlj, qij))
+                    tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
+                W(W_QLR, krel - 1) = R(qlj);
+                W(W_QIR, krel - 1) = R(qij);
+                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij);
+            } else if (k == kpen) {
+                bad = T.conden(R(in(a.ps0, k - 1)) + ppen, thlu_top, qtu_top, th, qvj, qlj, qij);
+            } else {
+                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij);
+            }
+            if (bad) tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
+            W(W_QLR, k) = R(qlj);
+            W(W_QIR, k) = R(qij);
+        }
+    }
+    tm.sync();
+
+    // ---- S14 fluxes of the penetrative entrainment; none from the cloud top up ----
+    if (run) {
+        for (int k = w; k <= mkx; k += nw) {
+            if (k < kbup) continue;
+            if (k <= kpen - 1) {
+                const R d = R(in(a.ps0, k) - in(a.p0, k));
+                const R emfk = W(W_EMF, k);
+                out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * emfk * (W(W_THLUE, k) - (Er(A_THL0, k) + Er(A_SSTHL0, k) * d)));
+                out(a.qtflx, k) = D(emfk * (W(W_QTUE, k) - (Er(A_QT0, k) + Er(A_SSQT0, k) * d)));
+                W(W_UFLX, k) = emfk * (W(W_UUE, k) - (R(in(a.u0, k)) + Er(A_SSU0, k) * d));
+                W(W_VFLX, k) = emfk * (W(W_VUE, k) - (R(in(a.v0, k)) + Er(A_SSV0, k) * d));
+                for (int m = kTrLimited; m <= ncnst; ++m)
+                    if (tr_moved(m)) WT(3, m, k) = emfk * (WT(2, m, k) - (R(trin(m, k)) + WT(0, m, k) * d));
+            } else {
+                out(a.slflx, k) = 0.0;
+                out(a.qtflx, k) = 0.0;
+                if (k == kpen) { W(W_UFLX, k) = R(0); W(W_VFLX, k) = R(0); }
+                for (int m = kTrLimited; m <= ncnst; ++m)
+                    if (tr_moved(m)) WT(3, m, k) = R(0);
+            }
+        }
+    }
+    tm.sync();
+    if (run) {
+        for (int k = w; k <= mkx; k += nw) {
+            if (k < 1) continue;
+            if (k <= kpen) {
+                out(a.uten, k) = D((W(W_UFLX, k - 1) - W(W_UFLX, k)) * g / R(in(a.dp0, k)));
+                out(a.vten, k) = D((W(W_VFLX, k - 1) - W(W_VFLX, k)) * g / R(in(a.dp0, k)));
+            } else {
+                out(a.uten, k) = 0.0;
+                out(a.vten, k) = 0.0;
+            }
+        }
+    }
+    tm.sync();
+
+    // ---- S15 subsidence condensate sinks, S16 tendencies (uwshcu.F90:3416-3794) ----
+    if (run) {
+        const R ps00 = R(in(a.ps0, 0)), psinv = R(in(a.ps0, kinv - 1));
+        auto uemf = [&](int k) -> R {   // uwshcu.F90:3416-3422
+            if (k <= kinv - 2) return cbmf * (ps00 - R(in(a.ps0, k))) / (ps00 - psinv);
+            if (k <= krel - 1) return cbmf;
+            if (k <= kbup - 1) return R(out(a.umf, k));
+            if (k <= kpen - 1) return W(W_EMF, k);
+            return R(0);
+        };
+        auto uf = [&](int k) -> R { return R(in(a.u0, k)) + R(out(a.uten, k)) * dt; };
+        auto vf = [&](int k) -> R { return R(in(a.v0, k)) + R(out(a.vten, k)) * dt; };
+        for (int k = w; k <= kpen; k += nw) {
+            if (k < 1) continue;
+            D th, qvj, qlj, qij;
+            const R comsub = R(0.5) * (uemf(k) + uemf(k - 1));
+            const R thl0k = Er(A_THL0, k), qt0k = Er(A_QT0, k), ql0k = R(in(a.ql0, k)), qi0k = R(in(a.qi0, k));
+            R thlten_sub, qtten_sub, qlten_sub, qiten_sub, nlten_sub, niten_sub;
+            if (comsub >= R(0)) {
+                if (k == mkx) {
+                    thlten_sub = qtten_sub = qlten_sub = qiten_sub = nlten_sub = niten_sub = R(0);
+                } else {
+                    const R dp = R(in(a.p0, k) - in(a.p0, k + 1));
+                    thlten_sub = g * comsub * (Er(A_THL0, k + 1) - thl0k) / dp;
+                    qtten_sub = g * comsub * (Er(A_QT0, k + 1) - qt0k) / dp;
+                    qlten_sub = g * comsub * (R(in(a.ql0, k + 1)) - ql0k) / dp;
+                    qiten_sub = g * comsub * (R(in(a.qi0, k + 1)) - qi0k) / dp;
+                    nlten_sub = g * comsub * (trz(ixl, k + 1) - trz(ixl, k)) / dp;
+                    niten_sub = g * comsub * (trz(ixi, k + 1) - trz(ixi, k)) / dp;
+                }
+            } else {
+                if (k == 1) {
+                    thlten_sub = qtten_sub = qlten_sub = qiten_sub = nlten_sub = niten_sub = R(0);
+                } else {
+                    const R dp = R(in(a.p0, k - 1) - in(a.p0, k));
+                    thlten_sub = g * comsub * (thl0k - Er(A_THL0, k - 1)) / dp;
+                    qtten_sub = g * comsub * (qt0k - Er(A_QT0, k - 1)) / dp;
+                    qlten_sub = g * comsub * (ql0k - R(in(a.ql0, k - 1))) / dp;
+                    qiten_sub = g * comsub * (qi0k - R(in(a.qi0, k - 1))) / dp;
+                    nlten_sub = g * comsub * (trz(ixl, k) - trz(ixl, k - 1)) / dp;
+                    niten_sub = g * comsub * (trz(ixi, k) - trz(ixi, k - 1)) / dp;
+                }
+            }
+            const R thl_prog = thl0k + thlten_sub * dt;
+            const R qt_prog = fmax(qt0k + qtten_sub * dt, R(1.e-12));
+            if (T.conden_x(in(a.p0, k), E(A_EXN0, k), thl_prog, qt_prog, th, qvj, qlj, qij))
+                tm.fail((k << 4) | EX_SUBCONDEN);
+            const R qlsink = fmax(qlten_sub, -ql0k / dt), qisink = fmax(qiten_sub, -qi0k / dt);
+            const R nlsink = fmax(nlten_sub, -trz(ixl, k) / dt), nisink = fmax(niten_sub, -trz(ixi, k) / dt);
+
+            const int km1 = k - 1;
+            const R dp0k = R(in(a.dp0, k));
+            const R umf_km1 = R(out(a.umf, k - 1)), umf_k = R(out(a.umf, k));
+            // below the release layer the plume arrays hold nothing of this column's plume
+            const R dwk = (k < krel ? R(0) : W(W_DWTEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
+            const R dik = (k < krel ? R(0) : W(W_DITEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
+            const R qrk = frc_rasn * dwk, qsk = frc_rasn * dik;
+            out(a.qrten, k) = D(qrk);
+            out(a.qsten, k) = D(qsk);
+            R slten = (R(out(a.slflx, km1)) - R(out(a.slflx, k))) * g / dp0k;
+            const R u0k = R(in(a.u0, k)), v0k = R(in(a.v0, k));
+            if (k == 1) {
+                slten = slten - g / R(4) / dp0k *
+                                    (W(W_UFLX, k) * (uf(k + 1) - uf(k) + R(in(a.u0, k + 1)) - u0k) +
+                                     W(W_VFLX, k) * (vf(k + 1) - vf(k) + R(in(a.v0, k + 1)) - v0k));
+            } else if (k >= 2 && k <= kpen - 1) {
+                slten = slten - g / R(4) / dp0k *
+                                    (W(W_UFLX, k) * (uf(k + 1) - uf(k) + R(in(a.u0, k + 1)) - u0k) +
+                                     W(W_UFLX, k - 1) * (uf(k) - uf(k - 1) + u0k - R(in(a.u0, k - 1))) +
+                                     W(W_VFLX, k) * (vf(k + 1) - vf(k) + R(in(a.v0, k + 1)) - v0k) +
+                                     W(W_VFLX, k - 1) * (vf(k) - vf(k - 1) + v0k - R(in(a.v0, k - 1))));
+            } else if (k == kpen) {
+                slten = slten - g / R(4) / dp0k *
+                                    (W(W_UFLX, k - 1) * (uf(k) - uf(k - 1) + u0k - R(in(a.u0, k - 1))) +
+                                     W(W_VFLX, k - 1) * (vf(k) - vf(k - 1) + v0k - R(in(a.v0, k - 1))));
+            }
+            const R qtten = (R(out(a.qtflx, km1)) - R(out(a.qtflx, k))) * g / dp0k;
+
+            R qlu_mid = R(0), qiu_mid = R(0), qlr = R(0), qir = R(0);
+            if (k >= krel) {
+                qlr = W(W_QLR, k);
+                qir = W(W_QIR, k);
+                const R qlubelow = W(W_QLR, k - 1), qiubelow = W(W_QIR, k - 1);
+                if (k == krel) {
+                    qlu_mid = R(0.5) * (qlubelow + qlr) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                    qiu_mid = R(0.5) * (qiubelow + qir) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                } else if (k == kpen) {
+                    qlu_mid = R(0.5) * (qlubelow + qlr) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                    qiu_mid = R(0.5) * (qiubelow + qir) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                } else {
+                    qlu_mid = R(0.5) * (qlubelow + qlr);
+                    qiu_mid = R(0.5) * (qiubelow + qir);
+                }
+            }
+
+            R qc_l = (R(1) - frc_rasn) * dwk;
+            R qc_i = (R(1) - frc_rasn) * dik;
+            R qc_lm, qc_im, nc_lm, nc_im;
+            if (k <= kbup) {
+                const R fdrk = k < krel ? R(0) : W(W_FDR, k);
+                qc_l = qc_l + g * R(0.5) * (umf_km1 + umf_k) * fdrk * qlu_mid;
+                qc_i = qc_i + g * R(0.5) * (umf_km1 + umf_k) * fdrk * qiu_mid;
+                qc_lm = -g * R(0.5) * (umf_km1 + umf_k) * fdrk * ql0k;
+                qc_im = -g * R(0.5) * (umf_km1 + umf_k) * fdrk * qi0k;
+                nc_lm = -g * R(0.5) * (umf_km1 + umf_k) * fdrk * trz(ixl, k);
+                nc_im = -g * R(0.5) * (umf_km1 + umf_k) * fdrk * trz(ixi, k);
+            } else {
+                qc_lm = R(0); qc_im = R(0); nc_lm = R(0); nc_im = R(0);
+            }
+            if (k == kbup) {
+                const R dps = R(in(a.ps0, k - 1) - in(a.ps0, k));
+                qc_l = qc_l + g * umf_k * qlr / dps;
+                qc_i = qc_i + g * umf_k * qir / dps;
+                qc_lm = qc_lm - g * umf_k * ql0k / dps;
+                qc_im = qc_im - g * umf_k * qi0k / dps;
+                nc_lm = nc_lm - g * umf_k * trz(ixl, k) / dps;
+                nc_im = nc_im - g * umf_k * trz(ixi, k) / dps;
+                D ql_e, qi_e;
+                if (T.conden_x(in(a.p0, k), E(A_EXN0, k), W(W_THLUE, k), W(W_QTUE, k), th, qvj, ql_e, qi_e))
+                    tm.fail((1 << 16) | (k << 4) | EX_KBUPCONDEN);
+                const R nl_e = (ql_e > 0.0 && has_nl) ? WT(2, ixl, k) : R(0);
+                const R ni_e = (qi_e > 0.0 && has_ni) ? WT(2, ixi, k) : R(0);
+                const R emfk = W(W_EMF, k);
+                qc_lm = qc_lm - g * emfk * (R(ql_e) - ql0k) / dps;
+                qc_im = qc_im - g * emfk * (R(qi_e) - qi0k) / dps;
+                nc_lm = nc_lm - g * emfk * (nl_e - trz(ixl, k)) / dps;
+                nc_im = nc_im - g * emfk * (ni_e - trz(ixi, k)) / dps;
+            }
+            const R qltenk = qc_l + frc_rasn * dwk + (fmax(R(0), ql0k + (qc_lm + qlsink) * dt) - ql0k) / dt;
+            const R qitenk = qc_i + frc_rasn * dik + (fmax(R(0), qi0k + (qc_im + qisink) * dt) - qi0k) / dt;
+            if (has_nl) trout(ixl, k) = D(fmax(nc_lm + nlsink, -trz(ixl, k) / dt));
+            if (has_ni) trout(ixi, k) = D(fmax(nc_im + nisink, -trz(ixi, k) / dt));
+            out(a.qlten, k) = D(qltenk);
+            out(a.qiten, k) = D(qitenk);
+            out(a.qvten, k) = D(qtten - qltenk - qitenk);
+            out(a.sten, k) = D(slten + xlv * qltenk + xls * qitenk);
+            W(W_QCL, k) = qc_l;
+            W(W_QCI, k) = qc_i;
+            out(a.qc, k) = D(qc_l + qc_i);
+            // for S17: the evaporation's rate but for the flux, and its limit
+            D es, qs;
+            T.qsat_es_qs(in_t0(k), in(a.p0, k), es, qs);
+            const R qv0k = R(in_qv0(k));
+            W(W_TRFD, k) = kevp * fmax((R(1) - qv0k / R(qs)), R(0));
+            W(W_TRFU, k) = fmax(R(0), (W(W_QW0, k) - qv0k) / dt);
+        }
+    }
+    tm.sync();
+
+    if (run && tm.failed() != 0x7fffffff) {
+        code = tm.failed() & 15;
+        run = false;
+    }
+    if (live && code != EX_NONE) {
+        // ---- the exits of S12, S15 and S16 ----
+        for (int k = w; k <= mkx; k += nw) zero_outputs_level(k);
+        if (lead) {
+            exit_scalars();
+            write_diag(0, code, final_pass ? 2 : 1, amb);
+            rstate(RS_CONT) = 0.0;
+        }
+    }
+
+    if (run) {
+        // ---- S17 precipitation evaporation (uwshcu.F90:3808-3934): from the cloud top down
+        // (above it there is no flux, and every term is zero) ----
+        if (lead) {
+            R rliq = R(0), rainflx = R(0), snowflx = R(0);
+            for (int k = 1; k <= kpen; ++k) {
+                const R dp0k = R(in(a.dp0, k));
+                rainflx = rainflx + R(out(a.qrten, k)) * dp0k / g;
+                snowflx = snowflx + R(out(a.qsten, k)) * dp0k / g;
+                rliq = rliq + R(out(a.qc, k)) * dp0k / g / R(1000);
+            }
+            R flxrain_k = R(0), flxsnow_k = R(0);   // fluxes at the top interface of layer k
+            R evpint_rain = R(0), evpint_snow = R(0);
+            for (int k = kpen; k >= 1; --k) {
+                const R dp0k = R(in(a.dp0, k));
+                const R t0k = R(in_t0(k));
+                const R rate = W(W_TRFD, k), evplimit = W(W_TRFU, k);
+                const R qrk = R(out(a.qrten, k)), qsk = R(out(a.qsten, k));
+                R snowmlt = (t0k > R(273.16)) ? fmax(R(0), flxsnow_k * g / dp0k) : R(0);
+                R evprain = rate * sqrt(flxrain_k + snowmlt * dp0k / g);
+                R evpsnow = rate * sqrt(fmax(flxsnow_k - snowmlt * dp0k / g, R(0)));
+                R evplimit_rain = fmin(evplimit, (flxrain_k + snowmlt * dp0k / g) * g / dp0k);
+                evplimit_rain = fmin(evplimit_rain, (rainflx - evpint_rain) * g / dp0k);
+                evprain = fmax(R(0), fmin(evplimit_rain, evprain));
+                R evplimit_snow = fmin(evplimit, fmax(flxsnow_k - snowmlt * dp0k / g, R(0)) * g / dp0k);
+                evplimit_snow = fmin(evplimit_snow, (snowflx - evpint_snow) * g / dp0k);
+                evpsnow = fmax(R(0), fmin(evplimit_snow, evpsnow));
+                if ((evprain + evpsnow) > evplimit) {
+                    const R tmp1 = evprain * evplimit / (evprain + evpsnow);
+                    const R tmp2 = evpsnow * evplimit / (evprain + evpsnow);
+                    evprain = tmp1;
+                    evpsnow = tmp2;
+                }
+                evpint_rain = evpint_rain + evprain * dp0k / g;
+                evpint_snow = evpint_snow + evpsnow * dp0k / g;
+                const R ntraprd = qrk - evprain + snowmlt;
+                const R ntsnprd = qsk - evpsnow - snowmlt;
+                const R flxrain_km1 = fmax(flxrain_k + ntraprd * dp0k / g, R(0));
+                const R flxsnow_km1 = fmax(flxsnow_k + ntsnprd * dp0k / g, R(0));
+                flxrain_k = flxrain_km1;
+                flxsnow_k = flxsnow_km1;
+                out(a.flxprc1, k - 1) = final_pass ? D(flxrain_km1 + flxsnow_km1) : D(0.0);
+                out(a.flxsnow1, k - 1) = final_pass ? D(flxsnow_km1) : D(0.0);
+                W(W_QLSINK, k) = evprain;
+                W(W_QISINK, k) = evpsnow;
+                W(W_NLSINK, k) = snowmlt;
+            }
+            cout(a.precip) = D((flxrain_k + flxsnow_k) / R(1000));
+            cout(a.snow) = D(flxsnow_k / R(1000));
+            cout(a.cbmf) = D(cbmf);
+            cout(a.rliq) = D(rliq);
+            cout(a.cnt) = D(mkx + 1 - kpen);
+            cout(a.cnb) = D(mkx + 1 - (krel - 1));
+            rstate(39) = (double)amb;
+            if (final_pass) {   // the implicit-CIN pass ends here
+                cout(a.cush) = rstate(0);
+                write_diag(2, 0, 2, amb);
+            }
+        }
+
+        // ---- S20 constituent limiter (uwshcu.F90:4007-4076), a constituent per thread; the
+        // downward transfers wait in the constituent's output until the upward sweep ----
+        for (int m = kTrLimited; m <= ncnst; ++m) {
+            if (!tr_moved(m) || m % nw != (nw - 1 - w)) continue;
+            const R trmin = R(C.qmin[m]);
+            const bool wet = C.wet[m] != 0;
+            auto pdelx = [&](int k) -> R { return wet ? R(in(a.dp0, k)) : R(in(a.dpdry0, k)); };
+            R below = R(0);   // trfd(k - 1)
+            for (int k = 1; k <= mkx - 1; ++k) {
+                const R dum = (R(trin(m, k)) - trmin) * pdelx(k) / g / dt + WT(3, m, k - 1) - WT(3, m, k) + below;
+                below = fmin(R(0), dum);
+                trout(m, k) = D(below);
+            }
+            R trfd_k = R(0), trfu_k = R(0);
+            for (int k = mkx; k >= 1; --k) {
+                const R trfd_km1 = k >= 2 ? R(trout(m, k - 1)) : R(0);
+                const R pk = pdelx(k), flx = WT(3, m, k - 1) - WT(3, m, k);
+                R trfu_km1 = R(0);
+                if (k >= 2) {
+                    const R dum = (R(trin(m, k)) - trmin) * pk / g / dt + WT(3, m, k - 1) - WT(3, m, k) + trfd_km1 - trfd_k - trfu_k;
+                    trfu_km1 = fmax(R(0), -dum);
+                }
+                trout(m, k) = D((flx + trfd_km1 - trfd_k + trfu_km1 - trfu_k) * g / pk);
+                trfd_k = trfd_km1;
+                trfu_k = trfu_km1;
+            }
+        }
+
+        // ---- S21 in-cloud diagnostics (uwshcu.F90:4092-4158), and the zeros of the levels
+        // outside the cloud ----
+        for (int k = w; k <= mkx; k += nw) {
+            if (k >= kpen) {
+                out(a.flxprc1, k) = 0.0;
+                out(a.flxsnow1, k) = 0.0;
+            }
+            if (k < 1) continue;
+            if (k > kpen) {
+                out(a.qrten, k) = 0.0;
+                out(a.qsten, k) = 0.0;
+                out(a.qc, k) = 0.0;
+                if (has_nl) trout(ixl, k) = 0.0;
+                if (has_ni) trout(ixi, k) = 0.0;
+            }
+            for (int m = 1; m <= ncnst && m < kTrLimited; ++m)
+                if (m != ixl && m != ixi) trout(m, k) = 0.0;
+            if (k < krel || k > kpen) {
+                out(a.cufrc, k) = 0.0;
+                out(a.qcu, k) = 0.0;
+                out(a.qlu, k) = 0.0;
+                out(a.qiu, k) = 0.0;
+                continue;
+            }
+            const R qlr = W(W_QLR, k), qir = W(W_QIR, k);
+            const R qlubelow = W(W_QLR, k - 1), qiubelow = W(W_QIR, k - 1), qcubelow = qlubelow + qiubelow;
+            R qcuk = R(0.5) * (qcubelow + qlr + qir);
+            R qluk = R(0.5) * (qlubelow + qlr);
+            R qiuk = R(0.5) * (qiubelow + qir);
+            R tmp2 = R(0), tmp3 = R(1);
+            if constexpr (ZW) {
+                if (a.zw.cloud_sh) {
+                    // zwshcu.F90:4412-4429: cumulus fraction widened by detrainment
+                    tmp3 = R(0.5) * R(a.zw.ufrc0);
+                    R tmp1 = (R(in(a.z0, k)) - R(in(a.z0, krel))) / (R(in(a.z0, kpen)) - R(in(a.z0, krel)) + R(10));
+                    tmp1 = R(1) + R(a.zw.ufrcz) * tmp1;
+                    tmp3 = tmp3 * tmp1;
+                    tmp2 = W(W_FDR, k) * R(out(a.umf, k)) * R(in(a.zs0, k) - in(a.zs0, k - 1)) * dt /
+                           R(in(a.dp0, k)) * R(9.8) * R(a.zw.ufrcd);
+                    tmp2 = fmin(R(1) - rmaxfrac, tmp2);
+                }
+            }
+            R cufrck;
+            if (k == krel) {
+                cufrck = (ufrclcl + W(W_UFRC, k)) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+            } else if (k == kpen) {
+                cufrck = (W(W_UFRC, k - 1) + R(0)) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                if ((qlr + qir) > criqc) {
+                    qcuk = R(0.5) * (qcubelow + criqc);
+                    qluk = R(0.5) * (qlubelow + criqc * qlr / (qlr + qir));
+                    qiuk = R(0.5) * (qiubelow + criqc * qir / (qlr + qir));
+                }
+            } else {
+                cufrck = (W(W_UFRC, k - 1) + W(W_UFRC, k));
+            }
+            out(a.qcu, k) = D(qcuk);
+            out(a.qlu, k) = D(qluk);
+            out(a.qiu, k) = D(qiuk);
+            if constexpr (ZW) cufrck = tmp3 * cufrck + tmp2;   // zwshcu.F90:4449
+            out(a.cufrc, k) = D(cufrck);
+        }
+    }
+    tm.sync();
+
+    // ---- S17's tendencies, S18 reserved condensate (uwshcu.F90:3966-3981) and S19 positive
+    // moisture, FP64 (uwshcu.F90:3995-4001, 5096-5162) ----
+    const double qvmin = C.qmin[1], qlmin = C.qmin[2], qimin = C.qmin[3];
+    unsigned adjusted = 0;   // this thread's levels (bit (k - w) / nw) that S19 changes
+    if (run) {
+        for (int k = w, bit = 0; k <= mkx; k += nw, ++bit) {
+            if (k < 1) continue;
+            D qvten = 0.0, qlten = 0.0, qiten = 0.0, sten = 0.0;
+            if (k <= kpen) {
+                const R evprain = W(W_QLSINK, k), evpsnow = W(W_QISINK, k), snowmlt = W(W_NLSINK, k);
+                const R qcl = W(W_QCL, k), qci = W(W_QCI, k);
+                out(a.evapc, k) = D(evprain + evpsnow);
+                const R qlt = R(out(a.qlten, k)) - R(out(a.qrten, k));
+                const R qit = R(out(a.qiten, k)) - R(out(a.qsten, k));
+                const R qvt = R(out(a.qvten, k)) + evprain + evpsnow;
+                const R st = R(out(a.sten, k)) - xlv * evprain - xls * evpsnow - (xls - xlv) * snowmlt;
+                qvten = D(qvt);
+                qlten = D(qlt - qcl);
+                qiten = D(qit - qci);
+                sten = D(st - (xls - xlv) * qci);
+            } else {
+                out(a.evapc, k) = 0.0;
+            }
+            out(a.qvten, k) = qvten;
+            out(a.qlten, k) = qlten;
+            out(a.qiten, k) = qiten;
+            out(a.sten, k) = sten;
+            const D ql = in(a.ql0, k) + qlten * dtd, qi = in(a.qi0, k) + qiten * dtd;
+            const D dql = fmax(0.0, 1.0 * qlmin - ql), dqi = fmax(0.0, 1.0 * qimin - qi);
+            const D qv = in_qv0(k) + qvten * dtd - dql - dqi;
+            if (1.0 * qvmin - qv > 0.0) tm.borrows();      // it borrows from the layer below
+            if (dql != 0.0 || dqi != 0.0) adjusted |= 1u << (bit & 31);
+        }
+    }
+    tm.sync();
+    if (!run) return;
+    const double xlvd = C.xlv, xlsd = C.xls;
+    if (!tm.borrowed()) {
+        // no layer runs dry: each level's own condensate adjustment
+        for (int k = w, bit = 0; k <= mkx; k += nw, ++bit) {
+            if (k < 1 || !(adjusted >> (bit & 31) & 1u)) continue;
+            D qvten = out(a.qvten, k), qlten = out(a.qlten, k), qiten = out(a.qiten, k), sten = out(a.sten, k);
+            const D ql = in(a.ql0, k) + qlten * dtd, qi = in(a.qi0, k) + qiten * dtd;
+            const D dql = fmax(0.0, 1.0 * qlmin - ql), dqi = fmax(0.0, 1.0 * qimin - qi);
+            out(a.qlten, k) = qlten + dql / dtd;
+            out(a.qiten, k) = qiten + dqi / dtd;
+            out(a.qvten, k) = qvten - (dql + dqi) / dtd;
+            out(a.sten, k) = sten + xlvd * (dql / dtd) + xlsd * (dqi / dtd);
+        }
+    } else if (lead) {
+        positive_moisture();
+    }
+}
+
+}  // namespace uwshcu
+#endif
