@@ -108,6 +108,10 @@ __global__ __launch_bounds__(256) void setup_kernel(FwdArgs args, int n, const u
                                                     const double* __restrict__ estbl) {
     __shared__ double s_estbl[UWSHCU_ESTBL_LEN];
     const int nvalid = valid_items(args, n);
+    if (STAGE == 1 && args.defer_mark) {   // all n marks, also of slots past a column map's end
+        const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+        if (t0 < n) args.defer_mark[t0] = 0;
+    }
     {   // whole workgroup past the listed columns (in one level row): nothing to do
         const long long t0 = (long long)blockIdx.x * blockDim.x;
         const long long j0 = t0 % n;
@@ -123,7 +127,6 @@ __global__ __launch_bounds__(256) void setup_kernel(FwdArgs args, int n, const u
     item_column(args, j, slot, col);
     const ThermoT<double, FAST> T{consts, s_estbl};
     const Column<R, double, ZW, FAST> c(args, T, col, slot);
-    if (STAGE == 1 && k == 0 && args.defer_mark) args.defer_mark[j] = 0;
     if (STAGE >= 3 && c.rstate(RS_CONT) == 0.0) return;   // it ended in its first pass
     if (STAGE == 1) c.setup_level1(k);
     else if (STAGE == 2) c.setup_level2(k);
