@@ -52,6 +52,8 @@ struct uwshcu_ctx {
     // columns whose second convection pass runs in a launch of its own
     int* d_defer = nullptr;
     double* d_defer_state = nullptr;   // NRESUME x defer_cols doubles: their saved scalars
+    double* d_rec = nullptr;           // environment records of the buoyancy sorting
+    size_t rec_bytes = 0;
     size_t defer_cols = 0;
     // chunk batching: the packed column range, its device tables and their pinned
     // host staging (reused once the event says the previous upload finished)
@@ -64,17 +66,26 @@ struct uwshcu_ctx {
     hipEvent_t ctab_event = nullptr;
     bool ctab_pending = false;
     hipStream_t stream = nullptr;
-    // this device's address of the static scratch array (uwshcu_forward_device_noalloc)
+    // this device's addresses of the static scratch arrays (uwshcu_forward_device_noalloc)
     void* d_scratch = nullptr;
+    void* d_scratch_lists = nullptr;
     std::mutex mu;
 };
 
 // Workspace of uwshcu_forward_device_noalloc: a fixed array in the code object's
 // device memory, one copy per GPU the library runs on, held until the process ends.
-// Host code never passes `scratch` itself to a kernel (on the host it is a stand-in,
-// not a device address): uwshcu_ctx_create looks up this device's address once with
-// hipGetSymbolAddress and every launch uses that.
+// Host code never passes the arrays themselves to a kernel (on the host they are stand-ins,
+// not device addresses): uwshcu_ctx_create looks up this device's addresses once with
+// hipGetSymbolAddress and every launch uses those.
 static __device__ __align__(256) unsigned char scratch[UWSHCU_NOALLOC_SCRATCH_BYTES];
+// And the lists, saved scalars and environment records of its split launch, for the most
+// columns whose workspace fits: at 3 levels and no constituents, where these take 0.63 of
+// the workspace's bytes per column (at 35 and 3, 0.31).
+constexpr size_t kNoallocColumns = UWSHCU_NOALLOC_SCRATCH_BYTES /
+                                   (4 * ((size_t)uwshcu::ENV_ARRAYS + uwshcu::WS_FIXED) * sizeof(double));
+constexpr size_t kNoallocListBytes = kNoallocColumns * (4 * (size_t)uwshcu::kEnvRecord + uwshcu::NRESUME) * sizeof(double) +
+                                     (kNoallocColumns * 4 + 64) * sizeof(int) + 2 * 256;
+static __device__ __align__(256) unsigned char scratch_lists[kNoallocListBytes];
 
 namespace {
 
@@ -113,20 +124,23 @@ double goff_gratch(double t, int itype, double tmelt) {
 
 bool hip_ok(hipError_t e) { return e == hipSuccess; }
 
-// Per-device address of `scratch`, looked up once per device with that device current.
+// Per-device addresses of `scratch` and `scratch_lists`, looked up once per device with that device current.
 constexpr int kMaxDevices = 64;
 std::mutex g_scratch_mu;
-void* g_scratch_addr[kMaxDevices] = {};
+void* g_scratch_addr[kMaxDevices][2] = {};
 
-int scratch_address(int device, void** out) {
+int scratch_address(int device, void** out, void** lists) {
     if (device < 0 || device >= kMaxDevices) return UWSHCU_ERR_ARG;
     std::lock_guard<std::mutex> lk(g_scratch_mu);
-    if (!g_scratch_addr[device]) {
-        void* p = nullptr;
+    if (!g_scratch_addr[device][1]) {
+        void *p = nullptr, *q = nullptr;
         if (!hip_ok(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch))) || !p) return UWSHCU_ERR_HIP;
-        g_scratch_addr[device] = p;
+        if (!hip_ok(hipGetSymbolAddress(&q, HIP_SYMBOL(scratch_lists))) || !q) return UWSHCU_ERR_HIP;
+        g_scratch_addr[device][0] = p;
+        g_scratch_addr[device][1] = q;
     }
-    *out = g_scratch_addr[device];
+    *out = g_scratch_addr[device][0];
+    *lists = g_scratch_addr[device][1];
     return UWSHCU_OK;
 }
 
@@ -190,10 +204,11 @@ struct ZwInputs {
 };
 
 // fixed_ws (nullable): run in this caller-given workspace of fixed_bytes instead of the
-// context's, allocating nothing (FP64 only, one batch, no deferred-column lists).
+// context's, and fixed_lists the lists, saved scalars and records: nothing is allocated
+// (FP64 only, one batch).
 int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pcols, int ncol, int pver, int ncnst,
                double dt, const Chunk& ch, int* diag, hipStream_t stream, const ZwInputs* zw = nullptr,
-               void* fixed_ws = nullptr, size_t fixed_bytes = 0) {
+               void* fixed_ws = nullptr, size_t fixed_bytes = 0, void* fixed_lists = nullptr) {
     if (!ctx || pcols < 1 || ncol < 0 || ncol > pcols || pver < 3 || ncnst < 0 || ncnst > UWSHCU_NCNST_MAX)
         return UWSHCU_ERR_ARG;
     if (precision != UWSHCU_FP64 && precision != UWSHCU_MIXED && precision != UWSHCU_MIXED_UNCHECKED &&
@@ -206,13 +221,14 @@ int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pco
     const bool recompute = precision == UWSHCU_MIXED;
     const size_t per_col = uwshcu_workspace_bytes_per_column(pver, ncnst, precision);
     const size_t per_col64 = uwshcu_workspace_bytes_per_column(pver, ncnst, UWSHCU_FP64);
+    const size_t rec_col = fp32 ? 0 : (size_t)(pver + 1) * uwshcu::kEnvRecord * sizeof(double);
     // batches of columns that share one workspace; a fixed workspace holds the whole
     // chunk (its leading dimension rounded up to a wavefront) or the call is refused
-    const long long nb = fixed_ws ? ((long long)ncol + 63) / 64 * 64 : batch_columns(ctx, ncol, per_col);
+    const long long nb = fixed_ws ? ((long long)ncol + 63) / 64 * 64 : batch_columns(ctx, ncol, per_col + rec_col);
     if (fixed_ws && per_col * (size_t)nb > fixed_bytes) return UWSHCU_ERR_SCRATCH;
     if (ncol == 0) return UWSHCU_OK;
     if (!hip_ok(hipSetDevice(ctx->device))) return UWSHCU_ERR_HIP;
-    const long long nb64 = recompute ? batch_columns(ctx, ncol, per_col64) : 0;
+    const long long nb64 = recompute ? batch_columns(ctx, ncol, per_col64 + rec_col) : 0;
     size_t need = per_col * (size_t)nb;
     if (recompute && per_col64 * (size_t)nb64 > need) need = per_col64 * (size_t)nb64;
     int rc = fixed_ws ? UWSHCU_OK : ensure_ws(ctx, need);
@@ -236,6 +252,18 @@ int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pco
             return UWSHCU_ERR_NOMEM;
         }
         ctx->defer_cols = (size_t)nb + 1;
+    }
+    // the buoyancy sorting's environment records
+    const size_t need_rec = fixed_ws ? 0 : rec_col * (size_t)nb;
+    if (need_rec > ctx->rec_bytes) {
+        if (ctx->d_rec) {
+            if (!hip_ok(hipDeviceSynchronize())) return UWSHCU_ERR_HIP;
+            (void)hipFree(ctx->d_rec);
+            ctx->d_rec = nullptr;
+            ctx->rec_bytes = 0;
+        }
+        if (!hip_ok(hipMalloc((void**)&ctx->d_rec, need_rec))) return UWSHCU_ERR_NOMEM;
+        ctx->rec_bytes = need_rec;
     }
 
     FwdArgs a{};
@@ -263,11 +291,20 @@ int run_device(uwshcu_ctx* ctx, int precision, const uwshcu_params* par, int pco
         a.tpert = zw->tpert;
         a.qpert = zw->qpert;
     }
-    if (!fixed_ws && ctx->d_defer && (size_t)nb + 1 <= ctx->defer_cols) {
-        a.defer_list = ctx->d_defer + 2;   // two counts, then the lists and marks (see launch_column_pipeline)
+    // defer_count: two counts, then the lists and marks (see launch_column_pipeline);
+    // defer_state: [field][slot], a.wld = nb apart
+    if (fixed_ws) {
+        a.rec = static_cast<double*>(fixed_lists);
+        a.defer_state = a.rec + (size_t)(pver + 1) * uwshcu::kEnvRecord * (size_t)nb;
+        a.defer_count = reinterpret_cast<int*>(a.defer_state + (size_t)uwshcu::NRESUME * (size_t)nb);
+        const size_t used = (size_t)((char*)(a.defer_count + 2 + uwshcu::defer_list_ints((size_t)nb)) - (char*)fixed_lists);
+        if (used > kNoallocListBytes) return UWSHCU_ERR_SCRATCH;
+    } else {
+        a.rec = ctx->d_rec;
+        a.defer_state = ctx->d_defer_state;
         a.defer_count = ctx->d_defer;
-        a.defer_state = ctx->d_defer_state;   // [field][slot], a.wld = nb apart
     }
+    a.defer_list = a.defer_count + 2;
     if (recompute) {
         // the FP32 pass overwrites cush; the FP64 recompute reads the input value
         if (!hip_ok(hipMemcpyAsync(ctx->d_cush_in, ch.cush, (size_t)ncol * sizeof(double), hipMemcpyDeviceToDevice,
@@ -618,7 +655,7 @@ int uwshcu_ctx_create(const uwshcu_consts* c, const double* estbl, int device, u
               hip_ok(hipMemcpy(ctx->d_consts, &ctx->consts, sizeof(uwshcu_consts), hipMemcpyHostToDevice)) &&
               hip_ok(hipMemcpy(ctx->d_estbl, ctx->estbl, sizeof(ctx->estbl), hipMemcpyHostToDevice)) &&
               hip_ok(uwshcu::launch_clear_status(ctx->d_err, nullptr)) && hip_ok(hipStreamCreate(&ctx->stream)) &&
-              scratch_address(device, &ctx->d_scratch) == UWSHCU_OK && hip_ok(hipDeviceSynchronize());
+              scratch_address(device, &ctx->d_scratch, &ctx->d_scratch_lists) == UWSHCU_OK && hip_ok(hipDeviceSynchronize());
     if (!ok) {
         uwshcu_ctx_destroy(ctx);
         return UWSHCU_ERR_HIP;
@@ -644,6 +681,7 @@ int uwshcu_ctx_destroy(uwshcu_ctx* ctx) {
     if (ctx->d_parcol) (void)hipFree(ctx->d_parcol);
     if (ctx->d_defer) (void)hipFree(ctx->d_defer);
     if (ctx->d_defer_state) (void)hipFree(ctx->d_defer_state);
+    if (ctx->d_rec) (void)hipFree(ctx->d_rec);
     if (ctx->d_packed) (void)hipFree(ctx->d_packed);
     if (ctx->d_ctab) (void)hipFree(ctx->d_ctab);
     if (ctx->h_ctab) (void)hipHostFree(ctx->h_ctab);
@@ -739,7 +777,7 @@ int uwshcu_forward_device_noalloc(uwshcu_ctx* ctx, const uwshcu_params* par, int
              umf, slflx, qtflx, flxprc1, flxsnow1, qvten, qlten, qiten, sten, uten, vten, trten,
              qrten, qsten, precip, snow, evapc, cufrc, qcu, qlu, qiu, cbmf, qc, rliq, cnt, cnb, wu};
     return run_device(ctx, UWSHCU_FP64, par, pcols, ncol, pver, ncnst, dt, ch, diag, (hipStream_t)stream, nullptr,
-                      ctx->d_scratch, UWSHCU_NOALLOC_SCRATCH_BYTES);
+                      ctx->d_scratch, UWSHCU_NOALLOC_SCRATCH_BYTES, ctx->d_scratch_lists);
 }
 
 int uwshcu_zw_forward_device(uwshcu_ctx* ctx, const uwshcu_params* par, const uwshcu_zw_params* zw, int pcols,

@@ -51,11 +51,17 @@ enum EnvArray : int {
 };
 // Plume and flux working arrays, in the bulk type R.
 enum WsArray : int {
-    W_EMF, W_THLU, W_QTU, W_UU, W_VU, W_THVU, W_UFRC, W_REI, W_FER, W_FDR, W_DWTEN, W_DITEN,
-    W_THLUE, W_QTUE, W_UUE, W_VUE, W_UFLX, W_VFLX, W_QLSINK, W_QISINK, W_NLSINK, W_NISINK,
+    W_THLU, W_QTU, W_UU, W_VU, W_REI, W_FDR, W_DWTEN, W_DITEN, W_UFRC, W_THVU, W_FER,   // or plume records
+    W_EMF, W_THLUE, W_QTUE, W_UUE, W_VUE, W_UFLX, W_VFLX, W_QLSINK, W_QISINK, W_NLSINK, W_NISINK,
     W_QCL, W_QCI, W_QW0, W_TRFD, W_TRFU, W_QLR, W_QIR,
     WS_FIXED
 };
+// On the GPU the FP64 split launches keep the buoyancy sorting's results of a level together:
+// the record of slot j, level k lies at (j (mkx+1) + k) kPlumeRecord of the memory of the
+// arrays W_THLU .. W_FER, fields W_THLU .. W_UFRC, then the mass flux and the velocity.
+// Lanes at levels of their own write and read whole cache lines of it.
+enum PlumeField : int { P_UMF = W_UFRC + 1, P_WU, kPlumeRecord };
+static_assert((int)kPlumeRecord == (int)W_FER + 1, "the records take the arrays' place");
 // Per-constituent blocks follow the fixed plume arrays: SSTR0, TRU, TRUE, TRFLX (ncnst arrays each).
 UWSHCU_HD inline int ws_arrays(int ncnst) { return WS_FIXED + 4 * ncnst; }
 // Workspace bytes per column: environment block of the FP64 type (d_size bytes per
@@ -96,6 +102,8 @@ struct FwdArgs {
     int* defer_list;
     int* defer_count;
     double* defer_state;
+    // optional: the environment of each level as one record (EnvLevelOf), slot by slot
+    double* rec;
     // 1 (with defer_list): a column that reaches the cloud-base closure of its first
     // pass stops there instead, saves its scalars and lists itself, so that only the
     // triggered columns run the convection stages, packed densely in a launch of their own
@@ -163,13 +171,13 @@ enum { kTrLimited = 4 };
 // so that each kernel holds only its own part's live state.
 enum : int {
     PART_ALL = 0,
-    PART_SORT = 1,      // a listed column from its closure (resume 1) or from the start of its
-                        // second pass (resume 2) through the buoyancy sorting (S11)
+    PART_SORT = 1,      // a listed column's buoyancy sorting (S11): sort_* (uwshcu_sort.h)
     PART_REST = 2,      // the same from the forcedCu filter (S12) through the in-cloud
                         // diagnostics (S21): rest_team (uwshcu_rest.h)
     PART_CLOSURE = 3,   // every column up to the cloud-base closure of its first pass
     PART_CIN2 = 4       // the same, after the level-parallel set-B environment (S22), through
-                        // the implicit-CIN iteration's CIN (S1-S7), deferring a second pass
+                        // the implicit-CIN iteration's CIN (S1-S7) and, where the column
+                        // convects a second time, that pass's closure (S8-S10)
 };
 
 enum { EX_NONE = 0, EX_CONDEN = 1, EX_KINV1 = 2, EX_KLCLMKX = 3, EX_KLFCMKX = 4, EX_MU3 = 5, EX_WTW = 6,
@@ -183,6 +191,41 @@ enum { EX_NONE = 0, EX_CONDEN = 1, EX_KINV1 = 2, EX_KLCLMKX = 3, EX_KLFCMKX = 4,
 // (scratch 1.2 KB -> 44 B per lane in the one-wavefront build).
 #define UW_INLINE __attribute__((always_inline))
 
+// The environment of layer k, and of its top interface, as the buoyancy sorting reads it.
+// With FwdArgs::rec, that of slot j lives at rec[(j (mkx+1) + k) kEnvRecord], 16-byte
+// aligned: lanes at levels of their own then read whole cache lines of it, where the
+// level-major arrays give each lane 8 bytes of a line per value (48 GB moved for 15 ms
+// of sorting at 1 036 800 x 35 x 3).  The first eight are what a level hands to the next.
+template <class D>
+struct EnvLevelOf {
+    D p0, dp0, exn0, thv0bot, thl0, qt0, u0, v0;
+    D thv0mid, qs0mid, z0, thv0top, ssthl, ssqt, ssu, ssv, ps0, exns0;
+};
+constexpr int kEnvRecord = 18;
+static_assert(sizeof(EnvLevelOf<double>) == kEnvRecord * sizeof(double), "a record is the struct");
+
+// One column's state in the buoyancy sorting (S11, uwshcu_sort.h).
+template <class R, class D>
+struct SortState {
+    // the release level's updraft, and the cloud-top height the iteration starts from
+    int krel = 0;
+    R prel = 0, thv0rel = 0, wlcl = 0;
+    D cush = 0;
+    int limit_ufrc = 0, limit_ppen = 0, amb = 0, exit_code = EX_NONE;
+    // the level loop: the next level, and the environment at its pressure pe
+    int iter = 0, k = 0, kbup = 0, kpen = 0, ktr = 0;
+    int kwu = 0;             // the highest level whose velocity an iteration has set
+    bool tr_mid = false;
+    R scaleh = 0, wtw = 0, pe = 0, dpe = 0, exne = 0, thvebot = 0, thle = 0, qte = 0, ue = 0, ve = 0, pe_tr = 0;
+    D exe = 0, dp0 = 0;   // dp0: of layer k
+    // the plume at interface k-1
+    R thlu = 0, qtu = 0, uu = 0, vu = 0, thvu = 0, wu = 0, umf = 0;
+    // the last level's, for the cloud top
+    R rho0j = 0, drage = 0, bogbot = 0, bogtop = 0, wtwb = 0;
+    R fer = 0, fer_krel = 0;
+    R ppen = 0, thlu_top = 0, qtu_top = 0;
+};
+
 // R: bulk (plume) arithmetic type; D: the FP64 type (double, or AD in the adjoint).
 // ZW: the modified scheme compute_zwshcu (zwshcu.F90:630-4969), FP64 only; its
 // differences from compute_uwshcu are marked where they apply.
@@ -192,6 +235,12 @@ struct Column {
     static_assert(!ZW || (std::is_same<R, double>::value && std::is_same<D, double>::value),
                   "the modified scheme runs in FP64");
     static constexpr bool kAD = is_ad<D>::value;
+    // the parts of a split launch use records (EnvLevelOf, PlumeField)
+#if defined(__HIP_DEVICE_COMPILE__)
+    static constexpr bool kRec = !kAD && std::is_same<R, double>::value;
+#else
+    static constexpr bool kRec = false;
+#endif
     const FwdArgs& a;
     const ThermoT<D, FAST>& T;
     const uwshcu_consts& C;
@@ -210,6 +259,12 @@ struct Column {
         if constexpr (kAD) ad_bind_tape(tape);
     }
 
+    // FwdArgs::rec of level k (16-byte pieces)
+    struct alignas(16) Pair { double x, y; };
+    UWSHCU_HD inline Pair* record(int k) const {
+        UW_CHECK(a.rec && k >= 0 && k <= mkx && iw >= 0 && (size_t)iw < wld);
+        return reinterpret_cast<Pair*>(a.rec + ((size_t)iw * KS + k) * kEnvRecord);
+    }
     // saved scalar f of a deferred column (FwdArgs::defer_state)
     UWSHCU_HD inline double& rstate(int f) const {
         UW_CHECK(f >= 0 && f < NRESUME && iw >= 0 && (size_t)iw < wld && a.defer_state);
@@ -307,6 +362,11 @@ struct Column {
     UWSHCU_HD inline R& W(int arr, int k) const {
         UW_CHECK(arr >= 0 && arr < WS_FIXED && k >= 0 && k <= mkx && iw >= 0 && (long long)iw < (long long)wld);
         return ws[((size_t)arr * KS + k) * wld + iw]; }
+    // plume field f (W_THLU .. W_UFRC) of level k: its record's, or its array's
+    UWSHCU_HD inline R& P(int f, int k) const {
+        if constexpr (kRec) return ws[((size_t)iw * KS + k) * kPlumeRecord + f];
+        else return W(f, k);
+    }
     UWSHCU_HD inline R& WT(int blk, int m, int k) const {   // blk 0..3, m 1-based
         UW_CHECK(blk >= 0 && blk < 4 && m >= 1 && m <= ncnst && k >= 0 && k <= mkx && iw >= 0 && (long long)iw < (long long)wld);
         return ws[((size_t)(WS_FIXED + blk * ncnst + (m - 1)) * KS + k) * wld + iw];
@@ -373,19 +433,26 @@ struct Column {
     UWSHCU_HD UW_INLINE bool env_mid(int k, D& thv0j, D& qs0) const {
         D& tv = E(E_THV0MID, k);
         if (tv == 0.0) {
-            D th, qv, ql, qi, es, qs;
-            if (T.conden_x(in(a.p0, k), E(A_EXN0, k), E(A_THL0, k), E(A_QT0, k), th, qv, ql, qi)) {
-                tv = -1.0;
-            } else {
-                tv = th * (1.0 + C.zvir * qv - ql - qi);
-                T.qsat_es_qs(E(A_THL0, k) * E(A_EXN0, k), in(a.p0, k), es, qs);
-                E(E_QS0MID, k) = qs;
-            }
+            D v, qs = 0.0;
+            env_mid_values(k, v, qs);
+            tv = v;
+            E(E_QS0MID, k) = qs;
         }
         thv0j = tv;
         qs0 = E(E_QS0MID, k);
         return tv > 0.0;
     }
+    UWSHCU_HD UW_INLINE void env_mid_values(int k, D& thv0j, D& qs0) const {
+        D th, qv, ql, qi, es;
+        if (T.conden_x(in(a.p0, k), E(A_EXN0, k), E(A_THL0, k), E(A_QT0, k), th, qv, ql, qi)) {
+            thv0j = -1.0;
+        } else {
+            thv0j = th * (1.0 + C.zvir * qv - ql - qi);
+            T.qsat_es_qs(E(A_THL0, k) * E(A_EXN0, k), in(a.p0, k), es, qs0);
+        }
+    }
+    // the launch keeps the environment's records: it reads the layer-mean saturation there
+    UWSHCU_HD inline bool keeps_records() const { return kRec; }
 
     // Before a pass.  In a split launch the stages that follow write every level of every
     // other output and read no working array at a level that they have not written; wu
@@ -529,6 +596,19 @@ struct Column {
         }
     }
 
+    // S11, one level at a time (uwshcu_sort.h): start iteration iter of the cloud-top height's
+    // three; one level, true while there is another; the end of an iteration; and a listed
+    // column's scalars at its start and end
+    UWSHCU_HD UW_INLINE EnvLevelOf<D> env_level_lower(int k) const;
+    UWSHCU_HD UW_INLINE EnvLevelOf<D> env_level_upper(int k) const;
+    UWSHCU_HD UW_INLINE EnvLevelOf<D> env_level(int k) const;
+    UWSHCU_HD UW_INLINE void sort_release(SortState<R, D>& q) const;
+    UWSHCU_HD UW_INLINE void sort_begin(SortState<R, D>& q, int iter) const;
+    UWSHCU_HD UW_INLINE bool sort_level(SortState<R, D>& q) const;
+    UWSHCU_HD UW_INLINE void sort_top(SortState<R, D>& q) const;
+    UWSHCU_HD UW_INLINE void sort_load(SortState<R, D>& q) const;
+    UWSHCU_HD UW_INLINE void sort_store(const SortState<R, D>& q, bool second_pass) const;
+
     // S12-S21 of a listed column, its levels shared by a team of threads (uwshcu_rest.h)
     template <class Team>
     UWSHCU_HD __attribute__((always_inline)) void rest_team(Team& tm, bool live, bool final_pass) const;
@@ -553,7 +633,7 @@ struct Column {
     // cache.  Every value equals the one run() computes itself without env_ready.
     UWSHCU_HD void setup_level1(int k) const {
         E(A_EXNS0, k) = upow(in(a.ps0, k) / C.p00, C.rovcp);
-        E(E_THV0MID, k) = 0.0;
+        if (!keeps_records()) E(E_THV0MID, k) = 0.0;
         if (k < 1) return;
         D qsp, enerr;
         const int doit = findsp_point(T, in_qv0(k), in_t0(k), in(a.p0, k), qsp, enerr);
@@ -566,7 +646,8 @@ struct Column {
         E(A_QT0, k) = qt0;
         E(A_THL0, k) = (t0 - C.xlv * ql0 / C.cp - C.xls * qi0 / C.cp) / E(A_EXN0, k);
     }
-    UWSHCU_HD void setup_level2(int k) const {
+    // Returns the level's record (EnvLevelOf; the caller keeps it or not).
+    UWSHCU_HD EnvLevelOf<D> setup_level2(int k) const {
         // minmod slope at level k as slope() computes it (the top level copies mkx-1)
         const int j = k < mkx ? k : mkx - 1;
         auto mm = [&](auto field) {
@@ -580,14 +661,19 @@ struct Column {
         E(A_SSU0, k) = mm([&](int q) { return in(a.u0, q); });
         E(A_SSV0, k) = mm([&](int q) { return in(a.v0, q); });
         for (int m = 1; m <= ncnst; ++m) {
+            if (!tr_entrained(m)) continue;
             const auto above = (R(trin(m, j + 1)) - R(trin(m, j))) / (R(in(a.p0, j + 1)) - R(in(a.p0, j)));
             const auto below = (j == 1) ? above
                                         : (R(trin(m, j)) - R(trin(m, j - 1))) / (R(in(a.p0, j)) - R(in(a.p0, j - 1)));
             WT(0, m, k) = (above > R(0)) ? fmax(R(0), fmin(above, below)) : fmin(R(0), fmax(above, below));
         }
         if (!interface_env_level(A_THL0, k)) E(A_THV0BOT, k) = -1.0;
-        D thv0j, qs0;
-        env_mid(k, thv0j, qs0);
+        D thv0j, qs0 = 0.0;
+        if (keeps_records()) env_mid_values(k, thv0j, qs0);
+        else env_mid(k, thv0j, qs0);
+        return EnvLevelOf<D>{in(a.p0, k), in(a.dp0, k), E(A_EXN0, k), E(A_THV0BOT, k), E(A_THL0, k), E(A_QT0, k),
+                             in(a.u0, k), in(a.v0, k), thv0j, qs0, in(a.z0, k), E(A_THV0TOP, k), E(A_SSTHL0, k),
+                             E(A_SSQT0, k), E(A_SSU0, k), E(A_SSV0, k), in(a.ps0, k), E(A_EXNS0, k)};
     }
 
     // S22 of a column's first pass, level-parallel (uwshcu.F90:4169-4329), after the
@@ -646,7 +732,8 @@ template <class R, class D, bool ZW, bool FAST>
 template <bool kSplit, int PART>
 UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body() const {
     static_assert(PART == PART_ALL || kSplit, "the parts of a split launch need the split build");
-    static_assert(PART != PART_REST, "S12-S21 of a split launch are rest_team");
+    static_assert(PART != PART_ALL || !kRec, "the whole column as one call has no records");
+    static_assert(PART != PART_SORT && PART != PART_REST, "S11 of a split launch is sort_*, S12-S21 rest_team");
     // what this launch continues from: 0 the start, 1 the closure of the first pass,
     // 2 the second convection pass, 4 the implicit-CIN iteration
     const int resume = PART == PART_CLOSURE ? 0 : PART == PART_CIN2 ? 4 : a.resume;
@@ -709,7 +796,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
     slope([&](int k) { return in(a.u0, k); }, A_SSU0);
     slope([&](int k) { return in(a.v0, k); }, A_SSV0);
     for (int k = 0; k <= mkx; ++k) E(E_THV0MID, k) = 0.0;
-    for (int m = 1; m <= ncnst; ++m) slope_tr([&](int k) { return R(trin(m, k)); }, m);
+    for (int m = 1; m <= ncnst; ++m)
+        if (tr_entrained(m)) slope_tr([&](int k) { return R(trin(m, k)); }, m);
     }
 
     // a column continued at its first pass keeps what launch 1 wrote; launch 1 of a split
@@ -733,9 +821,6 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
     D plcl = 0, plfc = 0, tkeavg = 0, thvlmin = 0, qtsrc = 0, thvlsrc = 0, thlsrc = 0, usrc = 0, vsrc = 0;
     D thv0lcl = 0, cin = 0, cinlcl = 0;
     R prel = 0, thv0rel = 0, cbmf = 0, wlcl = 0, ufrclcl = 0, ppen = 0, thlu_top = 0, qtu_top = 0;
-    R rho0j = 0, drage = 0, bogbot = 0, bogtop = 0, wtwb = 0;
-    R trsrc_tmp = 0;
-    (void)trsrc_tmp;
 
     // The scalars live across the split of a deferred column: every function-scope
     // local that the second convection pass reads or carries to the end of the column.
@@ -744,8 +829,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         io(0, cush); io(1, cin); io(2, cinlcl); io(3, plcl); io(4, plfc); io(5, tkeavg); io(6, thvlmin);
         io(7, qtsrc); io(8, thvlsrc); io(9, thlsrc); io(10, usrc); io(11, vsrc); io(12, thv0lcl); io(13, prel);
         io(14, thv0rel); io(15, cbmf); io(16, wlcl); io(17, ufrclcl); io(18, ppen); io(19, thlu_top);
-        io(20, qtu_top); io(21, rho0j); io(22, drage); io(23, bogbot); io(24, bogtop); io(25, wtwb); io(26, th);
-        io(27, qvj); io(28, qlj); io(29, qij); io(30, kinv); io(31, klcl); io(32, klfc); io(33, krel);
+        io(20, qtu_top);
+        io(30, kinv); io(31, klcl); io(32, klfc); io(33, krel);
         io(34, kbup); io(35, kpen); io(36, limit_ufrc); io(37, limit_ppen); io(38, limit_emf); io(39, amb);
         // the first pass's values that its implicit-CIN restore reads (a column continued
         // at its second pass has used them already)
@@ -796,7 +881,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         if (kSplit ? resume == iter : resume != 0) {
             // a deferred column continues with the scalars it saved: at the second pass
             // those of its implicit-CIN restore, whose convection starts afresh
-            if (!kSplit || iter == 2) start_pass(PART == PART_SORT);
+            if (!kSplit || iter == 2) zero_pass_state();
         } else {
         // ---- S1 kinv (uwshcu.F90:1455-1468) ----
         kinv = 1;
@@ -909,14 +994,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 kinv = kinv_o; klcl = klcl_o; klfc = klfc_o; plcl = plcl_o; plfc = plfc_o; tkeavg = tkeavg_o;
                 thvlmin = thvlmin_o; qtsrc = qtsrc_o; thvlsrc = thvlsrc_o; thlsrc = thlsrc_o; usrc = usrc_o;
                 vsrc = vsrc_o; thv0lcl = thv0lcl_o;
-                if (PART == PART_CIN2 ||
-                    (PART == PART_ALL && kSplit && (a.defer_list || a.defer_mark) && !a.defer_at_closure)) {
-                    // the second pass runs in a launch of its own: save, list, stop
-                    cush = tscaleh;
-                    defer_here(a.defer_mark != nullptr);
-                    return;
-                }
-                zero_pass_state();
+                if constexpr (!kRec) start_pass(PART == PART_CIN2);
             } else {
                 // iteration-1 outputs stand (uwshcu.F90:1897-2010): they are already in the
                 // output arrays; flxprc1/flxsnow1 were never written and stay zero.
@@ -929,10 +1007,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
 
         // From here on the environment is set A (the input state).
         {
-        R wtw;   // set by the closure, or at the start of the buoyancy sorting
         // a column continued at its first pass (resume 1) resumes at the buoyancy sorting
         if (kSplit ? !(resume == 1 && iter == 1) : true) {
-        if constexpr (PART == PART_CLOSURE) start_pass(true);
+        if constexpr (PART == PART_CLOSURE && !kRec) start_pass(true);
+        D winv_s = 0;                             // updraft velocity at the inversion
+        R thvu_rel = 0, uu_rel = 0, vu_rel = 0;   // and the plume at the release level
         // ---- S8 release level (uwshcu.F90:2035-2043) ----
         if (klcl < kinv) {
             krel = kinv;
@@ -954,8 +1033,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 if (a.zw.pertw) {
                     // zwshcu.F90:2282-2285: a warm perturbation widens the w' distribution
                     const double tp = fmin(a.tpert[i], a.zw.tpertmax);
-                    tkeavg = tkeavg + zmh_ramp(tp, 0.0, 2.0) * 2.0;
-                    sigmaw = sqrt(1.0 * tkeavg + 5.e-4) + zmh_ramp(tp, 0.0, 1.0) * 0.1;
+                    const D tke_warm = tkeavg + zmh_ramp(tp, 0.0, 2.0) * 2.0;
+                    sigmaw = sqrt(1.0 * tke_warm + 5.e-4) + zmh_ramp(tp, 0.0, 1.0) * 0.1;
                 }
                 if (a.zw.lf) {
                     // zwshcu.F90:2296-2300: ascent at the PBL-top layer lowers wcrit
@@ -998,20 +1077,15 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             cbmf = R(cbmf_d);
             wlcl = R(wlcl_d);
             ufrclcl = R(ufrclcl_d);
-            wtw = R(wtw_d);
-            for (int k = kinv - 1; k <= krel - 1; ++k) { out(a.umf, k) = cbmf_d; out(a.wu, k) = winv; }
+            winv_s = winv;
+            if constexpr (!kRec)
+                for (int k = kinv - 1; k <= krel - 1; ++k) { out(a.umf, k) = cbmf_d; out(a.wu, k) = winv; }
         }
         const R wrel = wlcl;
-        W(W_UFRC, krel - 1) = ufrclcl;
 
         // ---- S10 release-level updraft (uwshcu.F90:2205-2255) ----
-        W(W_EMF, krel - 1) = R(0);
-        out(a.umf, krel - 1) = D(cbmf);
-        out(a.wu, krel - 1) = D(wrel);
-        W(W_THLU, krel - 1) = R(thlsrc);
-        W(W_QTU, krel - 1) = R(qtsrc);
         if (T.conden(prel, thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-        W(W_THVU, krel - 1) = thv_of(th, qvj, qlj, qij);
+        thvu_rel = thv_of(th, qvj, qlj, qij);
         {
             R uplus = R(0), vplus = R(0);
             if (krel == kinv) {
@@ -1026,16 +1100,34 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 uplus = uplus + PGFc * Er(A_SSU0, krel) * (prel - R(in(a.ps0, krel - 1)));
                 vplus = vplus + PGFc * Er(A_SSV0, krel) * (prel - R(in(a.ps0, krel - 1)));
             }
-            W(W_UU, krel - 1) = R(usrc) + uplus;
-            W(W_VU, krel - 1) = R(vsrc) + vplus;
+            uu_rel = R(usrc) + uplus;
+            vu_rel = R(vsrc) + vplus;
+        }
+        if constexpr (!kRec) {
+            W(W_UFRC, krel - 1) = ufrclcl;
+            out(a.umf, krel - 1) = D(cbmf);
+            out(a.wu, krel - 1) = D(wrel);
+            W(W_THLU, krel - 1) = R(thlsrc);
+            W(W_QTU, krel - 1) = R(qtsrc);
+            W(W_THVU, krel - 1) = thvu_rel;
+            W(W_UU, krel - 1) = uu_rel;
+            W(W_VU, krel - 1) = vu_rel;
         }
         for (int m = kTrLimited; m <= ncnst; ++m) WT(1, m, krel - 1) = R(trin(m, 1));   // trsrc = tr0(1,m)
 
-        if (PART == PART_CLOSURE ||
-            (PART == PART_ALL && kSplit && iter == 1 && a.defer_at_closure && (a.defer_mark || a.defer_list))) {
-            // it convects: the plume stages run in a launch of their own, packed with the
-            // other columns that got this far
+        if (PART == PART_CLOSURE || PART == PART_CIN2) {
+            // it convects (a second time): the plume stages run in a launch of their own,
+            // packed with the other columns that got this far
             cush = tscaleh;
+            // the plume at the release level
+            rstate(21) = (double)val(R(thlsrc));
+            rstate(22) = (double)val(R(qtsrc));
+            rstate(23) = (double)val(uu_rel);
+            rstate(24) = (double)val(vu_rel);
+            rstate(25) = (double)val(thvu_rel);
+            rstate(26) = (double)val(wrel);
+            rstate(27) = (double)val(cbmf);
+            rstate(28) = (double)val(winv_s);
             defer_here(a.defer_mark != nullptr);
             return;
         }
@@ -1043,350 +1135,31 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
 
         // ---- S11 buoyancy sorting (uwshcu.F90:2296-2952) ----
         {
-        R scaleh = R(tscaleh);
-        if (R(tscaleh) < R(0)) scaleh = R(1000);
-        for (int iter_scaleh = 1; iter_scaleh <= 3; ++iter_scaleh) {
-            kbup = krel;
-            kpen = krel;
-            wtw = wlcl * wlcl;
-            R pe = R(0.5) * (prel + R(in(a.ps0, krel)));
-            R dpe = prel - R(in(a.ps0, krel));
-            D exe = T.exnf(D(pe));          // Exner function of pe, FP64
-            R exne = R(exe);
-            R thvebot = thv0rel;
-            R thle = Er(A_THL0, krel) + Er(A_SSTHL0, krel) * (pe - R(in(a.p0, krel)));
-            R qte = Er(A_QT0, krel) + Er(A_SSQT0, krel) * (pe - R(in(a.p0, krel)));
-            R ue = R(in(a.u0, krel)) + Er(A_SSU0, krel) * (pe - R(in(a.p0, krel)));
-            R ve = R(in(a.v0, krel)) + Er(A_SSV0, krel) * (pe - R(in(a.p0, krel)));
-            // tre(m) = tr0(krel,m) + sstr0(krel,m)*(pe - p0(krel)) is recomputed where used
-            R pe_tr = pe - R(in(a.p0, krel));
-            int ktr = krel;            // layer whose (tr0, sstr0) define tre, and offset pe_tr
-            bool tr_mid = false;       // after the first layer tre = tr0(k) exactly
-            // The plume at interface k-1: read from the workspace for the first level, then
-            // carried over from the level below, which stored the same values.
-            R c_thlu = W(W_THLU, krel - 1), c_qtu = W(W_QTU, krel - 1), c_uu = W(W_UU, krel - 1);
-            R c_vu = W(W_VU, krel - 1), c_thvu = W(W_THVU, krel - 1);
-            R c_wu = R(out(a.wu, krel - 1)), c_umf = R(out(a.umf, krel - 1));
-
-            for (int k = krel; k <= mkx - 1; ++k) {
-                const int km1 = k - 1;
-                // Read once for both iter_xc passes: the environment of layer k, which the loop
-                // body does not write, and (issued early) that of layer k+1 for the next level.
-                const R thlu_km1 = c_thlu, qtu_km1 = c_qtu;
-                const R uu_km1 = c_uu, vu_km1 = c_vu, thvu_km1 = c_thvu;
-                const R wu_km1 = c_wu;
-                const R z0k = R(in(a.z0, k)), dp0k = R(in(a.dp0, k)), thv0top_k = Er(A_THV0TOP, k);
-                const R ss_thl = Er(A_SSTHL0, k), ss_qt = Er(A_SSQT0, k), ss_u = Er(A_SSU0, k), ss_v = Er(A_SSV0, k);
-                const D ps0k = in(a.ps0, k), exns0k = E(A_EXNS0, k);
-                const D p0_kp1 = in(a.p0, k + 1), dp0_kp1 = in(a.dp0, k + 1), exn0_kp1 = E(A_EXN0, k + 1);
-                const R thv0bot_kp1 = Er(A_THV0BOT, k + 1), thl0_kp1 = Er(A_THL0, k + 1), qt0_kp1 = Er(A_QT0, k + 1);
-                const D u0_kp1 = in(a.u0, k + 1), v0_kp1 = in(a.v0, k + 1);
-                R thlue = thlu_km1;
-                R qtue = qtu_km1;
-                R wue = wu_km1;
-                wtwb = wtw;
-                const R umf_km1 = c_umf;
-                R umfk = 0, ferk = 0, fdrk = 0;
-                // Level-k results of an iter_xc pass.  Each pass overwrites the last and none
-                // reads them back, so they are stored once, after the passes.
-                R reik = 0, thluk = 0, qtuk = 0, uuk = 0, vuk = 0, thvuk = 0, dwtenk = 0, ditenk = 0;
-                // the environment at pe does not change between the iter_xc passes
-                R thv0j;
-                D es, qs;
-                if (k == krel) {
-                    if (T.conden_x(pe, exe, thle, qte, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                    thv0j = thv_of(th, qvj, qlj, qij);
-                    T.qsat_es_qs(D(thle * exne), pe, es, qs);
-                } else {
-                    D tv;
-                    if (!env_mid(k, tv, qs)) { exit_code = EX_CONDEN; goto L333; }
-                    thv0j = R(tv);
-                }
-                rho0j = pe / (r * thv0j * exne);
-                const R excess0 = qte - R(qs);
-                for (int iter_xc = 1; iter_xc <= 2; ++iter_xc) {
-                    wtw = wu_km1 * wu_km1;
-                    if (T.conden_x(pe, exe, thlue, qtue, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                    near(qlj + qij - criqc, criqc);
-                    if ((R(qlj) + R(qij)) > criqc) {
-                        const R qlr = R(qlj), qir = R(qij);
-                        const R exql = ((qlr + qir) - criqc) * qlr / (qlr + qir);
-                        const R exqi = ((qlr + qir) - criqc) * qir / (qlr + qir);
-                        qtue = qtue - exql - exqi;
-                        thlue = thlue + (xlv / cp / exne) * exql + (xls / cp / exne) * exqi;
-                        // unchanged arguments give unchanged results, so only re-adjust here
-                        if (T.conden_x(pe, exe, thlue, qtue, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                    }
-                    const R thvj = thv_of(th, qvj, qlj, qij);
-                    T.qsat_es_qs(D(thlue * exne), pe, es, qs);
-                    const R excessu = qtue - R(qs);
-                    near(excessu, qtue);
-                    near(excess0, qte);
-                    const R cridis = rle * scaleh;
-                    R xc;
-                    if ((excessu <= R(0) && excess0 <= R(0)) || (excessu >= R(0) && excess0 >= R(0))) {
-                        xc = fmin(R(1), fmax(R(0), R(1) - R(2) * rbuoy * g * cridis / (wue * wue) * (R(1) - thvj / thv0j)));
-                    } else {
-                        const R xsat = excessu / (excessu - excess0);
-                        const R thlxsat = thlue + xsat * (thle - thlue);
-                        const R qtxsat = qtue + xsat * (qte - qtue);
-                        if (T.conden_x(pe, exe, thlxsat, qtxsat, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                        const R thvxsat = thv_of(th, qvj, qlj, qij);
-                        R x_cu = 0, x_en = 0;
-                        for (int kk = 1; kk <= 2; ++kk) {
-                            R thv_x0, thv_x1;
-                            if (kk == 1) {
-                                thv_x0 = thvj;
-                                thv_x1 = (R(1) - R(1) / xsat) * thvj + (R(1) / xsat) * thvxsat;
-                            } else {
-                                thv_x1 = thv0j;
-                                thv_x0 = (xsat / (xsat - R(1))) * thv0j + (R(1) / (R(1) - xsat)) * thvxsat;
-                            }
-                            const R aquad = wue * wue;
-                            const R bquad = R(2) * rbuoy * g * cridis * (thv_x1 - thv_x0) / thv0j - R(2) * (wue * wue);
-                            const R cquad = R(2) * rbuoy * g * cridis * (thv_x0 - thv0j) / thv0j + (wue * wue);
-                            R xs1 = 0, xs2 = 0;
-                            int status;
-                            near(bquad * bquad - R(4) * aquad * cquad, bquad * bquad + fabs(R(4) * aquad * cquad));
-                            if (kk == 1) {
-                                if ((bquad * bquad - R(4) * aquad * cquad) >= R(0)) {
-                                    roots(aquad, bquad, cquad, xs1, xs2, status);
-                                    near(xsat - fmin(xs1, xs2), R(1));
-                                    x_cu = fmin(R(1), fmax(R(0), fmin(xsat, fmin(xs1, xs2))));
-                                } else {
-                                    x_cu = xsat;
-                                }
-                            } else {
-                                if ((bquad * bquad - R(4) * aquad * cquad) >= R(0)) {
-                                    roots(aquad, bquad, cquad, xs1, xs2, status);
-                                    x_en = fmin(R(1), fmax(R(0), fmax(xsat, fmin(xs1, xs2))));
-                                } else {
-                                    x_en = R(1);
-                                }
-                            }
-                        }
-                        xc = (x_cu == xsat) ? fmax(x_cu, x_en) : x_cu;
-                    }
-                    near(xc - R(0.5), R(1));
-                    const R ee2 = xc * xc;
-                    const R ud2 = R(1) - R(2) * xc + xc * xc;
-                    reik = (R(0.5) * rkm / z0k / g / rho0j);
-                    if (xc > R(0.5))
-                        reik = fmin(reik, R(0.9) * ulog(dp0k / g / dt / umf_km1 + R(1)) / dpe / (R(2) * xc - R(1)));
-                    ferk = reik * ee2;
-                    fdrk = reik * ud2;
-                    if constexpr (ZW) {
-                        if (a.zw.ent) {
-                            // zwshcu.F90:2818-2844: entrainment from the updraft buoyancy
-                            const R bog = rbuoy * (thvu_km1 / thvebot - R(1)) * g;
-                            ferk = R(a.zw.ent0) * bog / fmax(wue * wue, R(1.0e-4));
-                            const R fer_min = bog > R(1.e-4) ? R(1.e-4) : R(0);
-                            ferk = fmin(fmax(ferk, fer_min), R(3.0e-2));
-                        }
-                    }
-                    umfk = umf_km1 * uexp(dpe * (ferk - fdrk));
-                    if (ferk * dpe < R(1.e-4)) {
-                        thluk = thlu_km1 + (thle + ss_thl * dpe / R(2) - thlu_km1) * ferk * dpe;
-                        qtuk = qtu_km1 + (qte + ss_qt * dpe / R(2) - qtu_km1) * ferk * dpe;
-                        uuk = uu_km1 + (ue + ss_u * dpe / R(2) - uu_km1) * ferk * dpe - PGFc * ss_u * dpe;
-                        vuk = vu_km1 + (ve + ss_v * dpe / R(2) - vu_km1) * ferk * dpe - PGFc * ss_v * dpe;
-                    } else {
-                        const R ef = uexp(-ferk * dpe);
-                        thluk = (thle + ss_thl / ferk - ss_thl * dpe / R(2)) -
-                                (thle + ss_thl * dpe / R(2) - thlu_km1 + ss_thl / ferk) * ef;
-                        qtuk = (qte + ss_qt / ferk - ss_qt * dpe / R(2)) -
-                               (qte + ss_qt * dpe / R(2) - qtu_km1 + ss_qt / ferk) * ef;
-                        uuk = (ue + (R(1) - PGFc) * ss_u / ferk - ss_u * dpe / R(2)) -
-                              (ue + ss_u * dpe / R(2) - uu_km1 + (R(1) - PGFc) * ss_u / ferk) * ef;
-                        vuk = (ve + (R(1) - PGFc) * ss_v / ferk - ss_v * dpe / R(2)) -
-                              (ve + ss_v * dpe / R(2) - vu_km1 + (R(1) - PGFc) * ss_v / ferk) * ef;
-                    }
-                    if (T.conden_x(ps0k, exns0k, thluk, qtuk, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                    near(qlj + qij - criqc, criqc);
-                    if ((R(qlj) + R(qij)) > criqc) {
-                        const R qlr = R(qlj), qir = R(qij);
-                        const R exql = ((qlr + qir) - criqc) * qlr / (qlr + qir);
-                        const R exqi = ((qlr + qir) - criqc) * qir / (qlr + qir);
-                        qtuk = qtuk - exql - exqi;
-                        thluk = thluk + (xlv / cp / R(exns0k)) * exql + (xls / cp / R(exns0k)) * exqi;
-                        dwtenk = exql;
-                        ditenk = exqi;
-                        if (T.conden_x(ps0k, exns0k, thluk, qtuk, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                    } else {
-                        dwtenk = R(0);
-                        ditenk = R(0);
-                    }
-                    thvuk = thv_of(th, qvj, qlj, qij);
-                    bogbot = rbuoy * (thvu_km1 / thvebot - R(1));
-                    bogtop = rbuoy * (thvuk / thv0top_k - R(1));
-                    const R delbog = bogtop - bogbot;
-                    drage = ferk * (R(1) + rdrag);
-                    const R expfac = uexp(R(-2) * drage * dpe);
-                    wtwb = wtw;
-                    if (drage * dpe > R(1.e-3))
-                        wtw = wtw * expfac + (delbog + (R(1) - expfac) * (bogbot + delbog / (R(-2) * drage * dpe))) / (rho0j * drage);
-                    else
-                        wtw = wtw + dpe * (bogbot + bogtop) / rho0j;
-                    near(wtw, wtwb);
-                    near(bogtop, R(1));
-                    if (wtw > R(0)) {
-                        thlue = R(0.5) * (thlu_km1 + thluk);
-                        qtue = R(0.5) * (qtu_km1 + qtuk);
-                        wue = R(0.5) * sqrt(fmax(wtwb + wtw, R(0)));
-                    } else {
-                        break;   // go to 111
-                    }
-                }
-                // 111 continue
-                W(W_REI, k) = reik;
-                W(W_FER, k) = ferk;
-                W(W_FDR, k) = fdrk;
-                W(W_EMF, k) = R(0);
-                W(W_DWTEN, k) = dwtenk;
-                W(W_DITEN, k) = ditenk;
-                W(W_THLU, k) = thluk;
-                W(W_QTU, k) = qtuk;
-                W(W_UU, k) = uuk;
-                W(W_VU, k) = vuk;
-                out(a.umf, k) = D(umfk);
-                W(W_THVU, k) = thvuk;
-                // Updraft tracers (uwshcu.F90:2592-2614).  Nothing in an iter_xc pass reads
-                // them and each pass overwrites the last, so they are formed once, from the
-                // fer(k) of the pass that ended the loop.
-                if (ncnst < kTrLimited) {
-                } else if (ferk * dpe < R(1.e-4)) {
-                    for (int m = kTrLimited; m <= ncnst; ++m) {
-                        if (!tr_moved(m)) continue;
-                        const R tre = tr_mid ? R(trin(m, ktr)) : R(trin(m, ktr)) + WT(0, m, ktr) * pe_tr;
-                        WT(1, m, k) = WT(1, m, km1) + (tre + WT(0, m, k) * dpe / R(2) - WT(1, m, km1)) * ferk * dpe;
-                    }
-                } else {
-                    const R ef = uexp(-ferk * dpe);
-                    for (int m = kTrLimited; m <= ncnst; ++m) {
-                        if (!tr_moved(m)) continue;
-                        const R tre = tr_mid ? R(trin(m, ktr)) : R(trin(m, ktr)) + WT(0, m, ktr) * pe_tr;
-                        const R sst = WT(0, m, k);
-                        WT(1, m, k) = (tre + sst / ferk - sst * dpe / R(2)) -
-                                      (tre + sst * dpe / R(2) - WT(1, m, km1) + sst / ferk) * ef;
-                    }
-                }
-                if (umfk == R(0)) wtw = R(-1);
-                if (bogtop > R(0) && wtw > R(0)) kbup = k;
-                if (wtw <= R(0)) { kpen = k; break; }   // go to 45
-                {
-                    const R wuk = sqrt(wtw);
-                    out(a.wu, k) = D(wuk);
-                    if (wuk > R(100)) { exit_code = EX_WU; goto L333; }
-                    const R rhos0j = R(ps0k) / (r * R(0.5) * (thv0bot_kp1 + thv0top_k) * R(exns0k));
-                    R ufrck = umfk / (rhos0j * wuk);
-                    near(ufrck - rmaxfrac, rmaxfrac);
-                    if (ufrck > rmaxfrac) {
-                        limit_ufrc = 1;
-                        ufrck = rmaxfrac;
-                        umfk = rmaxfrac * rhos0j * wuk;
-                        out(a.umf, k) = D(umfk);
-                        W(W_FDR, k) = ferk - ulog(umfk / umf_km1) / dpe;
-                    }
-                    W(W_UFRC, k) = ufrck;
-                    c_wu = R(D(wuk));
-                    c_umf = R(D(umfk));
-                }
-                c_thlu = thluk;
-                c_qtu = qtuk;
-                c_uu = uuk;
-                c_vu = vuk;
-                c_thvu = thvuk;
-                pe = R(p0_kp1);
-                dpe = R(dp0_kp1);
-                exne = R(exn0_kp1);
-                if constexpr (sizeof(R) == sizeof(double)) exe = exn0_kp1;   // = exnf(pe), pe = p0(k+1)
-                else exe = T.exnf(D(pe));
-                thvebot = thv0bot_kp1;
-                thle = thl0_kp1;
-                qte = qt0_kp1;
-                ue = R(u0_kp1);
-                ve = R(v0_kp1);
-                ktr = k + 1;
-                tr_mid = true;
+            SortState<R, D> q;
+            q.krel = krel;
+            q.prel = prel;
+            q.thv0rel = thv0rel;
+            q.wlcl = wlcl;
+            q.cush = tscaleh;
+            q.limit_ufrc = limit_ufrc;
+            q.limit_ppen = limit_ppen;
+            q.amb = amb;
+            for (int iter_scaleh = 1; iter_scaleh <= 3 && !q.exit_code; ++iter_scaleh) {
+                sort_begin(q, iter_scaleh);
+                while (sort_level(q)) {}
+                if (!q.exit_code) sort_top(q);
             }
-            // 45 continue
-            if (drage == R(0)) {
-                const R aquad = (bogtop - bogbot) / R(in(a.ps0, kpen) - in(a.ps0, kpen - 1));
-                const R bquad = R(2) * bogbot;
-                const R wuk = R(out(a.wu, kpen - 1));
-                const R cquad = -(wuk * wuk) * rho0j;
-                R xc1 = 0, xc2 = 0;
-                int status;
-                roots(aquad, bquad, cquad, xc1, xc2, status);
-                const R dpk = R(in(a.dp0, kpen));
-                if (status == 0) {
-                    if (xc1 <= R(0) && xc2 <= R(0)) {
-                        ppen = fmax(xc1, xc2);
-                        ppen = fmin(R(0), fmax(-dpk, ppen));
-                    } else if (xc1 > R(0) && xc2 > R(0)) {
-                        ppen = -dpk;
-                    } else {
-                        ppen = fmin(xc1, xc2);
-                        ppen = fmin(R(0), fmax(-dpk, ppen));
-                    }
-                } else {
-                    ppen = -dpk;
-                }
-            } else {
-                ppen = compute_ppen(wtwb, drage, bogbot, bogtop, rho0j, R(in(a.dp0, kpen)));
-            }
-            if (ppen == -R(in(a.dp0, kpen)) || ppen == R(0)) limit_ppen = 1;
-            {
-                const R ferp = W(W_FER, kpen), thl0p = Er(A_THL0, kpen), ssthlp = Er(A_SSTHL0, kpen);
-                const R qt0p = Er(A_QT0, kpen), ssqtp = Er(A_SSQT0, kpen);
-                if (ferp * (-ppen) < R(1.e-4)) {
-                    thlu_top = W(W_THLU, kpen - 1) + (thl0p + ssthlp * (-ppen) / R(2) - W(W_THLU, kpen - 1)) * ferp * (-ppen);
-                    qtu_top = W(W_QTU, kpen - 1) + (qt0p + ssqtp * (-ppen) / R(2) - W(W_QTU, kpen - 1)) * ferp * (-ppen);
-                } else {
-                    const R ef = uexp(-ferp * (-ppen));
-                    thlu_top = (thl0p + ssthlp / ferp - ssthlp * (-ppen) / R(2)) -
-                               (thl0p + ssthlp * (-ppen) / R(2) - W(W_THLU, kpen - 1) + ssthlp / ferp) * ef;
-                    qtu_top = (qt0p + ssqtp / ferp - ssqtp * (-ppen) / R(2)) -
-                              (qt0p + ssqtp * (-ppen) / R(2) - W(W_QTU, kpen - 1) + ssqtp / ferp) * ef;
-                }
-            }
-            {
-                const R ptop = R(in(a.ps0, kpen - 1)) + ppen;
-                if (T.conden(ptop, thlu_top, qtu_top, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
-                near(qlj + qij - criqc, criqc);
-                const R exntop = R(upow(D(ptop) / C.p00, C.rovcp));
-                if ((R(qlj) + R(qij)) > criqc) {
-                    const R qlr = R(qlj), qir = R(qij);
-                    const R dw = ((qlr + qir) - criqc) * qlr / (qlr + qir);
-                    const R di = ((qlr + qir) - criqc) * qir / (qlr + qir);
-                    W(W_DWTEN, kpen) = dw;
-                    W(W_DITEN, kpen) = di;
-                    qtu_top = qtu_top - dw - di;
-                    thlu_top = thlu_top + (xlv / cp / exntop) * dw + (xls / cp / exntop) * di;
-                } else {
-                    W(W_DWTEN, kpen) = R(0);
-                    W(W_DITEN, kpen) = R(0);
-                }
-                const R rhos0j = R(in(a.ps0, kpen - 1)) / (r * R(0.5) * (Er(A_THV0BOT, kpen) + Er(A_THV0TOP, kpen - 1)) * Er(A_EXNS0, kpen - 1));
-                cush = D(R(in(a.zs0, kpen - 1)) - ppen / rhos0j / g);
-                scaleh = R(cush);
-            }
+            kbup = q.kbup;
+            kpen = q.kpen;
+            limit_ufrc = q.limit_ufrc;
+            limit_ppen = q.limit_ppen;
+            amb = q.amb;
+            if (q.exit_code) { exit_code = q.exit_code; goto L333; }
+            cush = q.cush;
+            ppen = q.ppen;
+            thlu_top = q.thlu_top;
+            qtu_top = q.qtu_top;
         }
-        if constexpr (PART == PART_SORT) {
-            // the rest of the pass runs in the next launch: save what S11 set (the other
-            // saved scalars still hold the closure's values, but for a second pass, whose
-            // closure ran here)
-            resume_io([&](int f, auto& x) {
-                const bool set_here = f == 0 || (f >= 18 && f <= 20) || (f >= 34 && f <= 37) || f == 39;
-                const bool closure = iter == 2 && ((f >= 13 && f <= 17) || f == 33);
-                if (!set_here && !closure) return;
-                if constexpr (std::is_integral<std::remove_reference_t<decltype(x)>>::value) rstate(f) = (double)x;
-                else rstate(f) = (double)val(x);
-            });
-            rstate(RS_CONT) = 1.0;
-            return;
-        }
-        }   // S11
 
         // ---- S12 forcedCu filter (uwshcu.F90:2964-2992) ----
         if (kbup == krel) { exit_code = EX_CUFILTER; goto L333; }
@@ -1866,7 +1639,6 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
 L333:
     write_exit();
     path = 0;
-    if constexpr (PART == PART_SORT) rstate(RS_CONT) = 0.0;
 
 Ldone:
     if (a.amb_flag) a.amb_flag[i] = amb;
@@ -1882,13 +1654,23 @@ Ldone:
 }  // namespace uwshcu
 
 #include "uwshcu_rest.h"
+#include "uwshcu_sort.h"
 
 namespace uwshcu {
 
 template <class R, class D, bool ZW, bool FAST>
 template <int PART>
 UWSHCU_HD void Column<R, D, ZW, FAST>::run_part() const {
-    if constexpr (PART == PART_REST) {
+    if constexpr (PART == PART_SORT) {
+        SortState<R, D> q;
+        sort_load(q);
+        for (int iter_scaleh = 1; iter_scaleh <= 3 && !q.exit_code; ++iter_scaleh) {
+            sort_begin(q, iter_scaleh);
+            while (sort_level(q)) {}
+            if (!q.exit_code) sort_top(q);
+        }
+        sort_store(q, false);
+    } else if constexpr (PART == PART_REST) {
         SerialTeam one;
         rest_team(one, true, false);
     } else {

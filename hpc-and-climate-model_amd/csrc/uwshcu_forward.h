@@ -27,7 +27,7 @@ __device__ inline void item_column(const FwdArgs& args, int j, int& slot, int& c
 }
 
 // One thread per column; the saturation table is staged into LDS once per workgroup.
-template <class R, bool ZW, bool SPLIT, bool FAST, int PART = PART_ALL>
+template <class R, bool ZW, bool FAST, int PART>
 __device__ __forceinline__ void forward_body(const FwdArgs& args, int n, const uwshcu_consts* __restrict__ consts,
                                              const double* __restrict__ estbl) {
     __shared__ double s_estbl[UWSHCU_ESTBL_LEN];
@@ -41,15 +41,7 @@ __device__ __forceinline__ void forward_body(const FwdArgs& args, int n, const u
     item_column(args, j, slot, col);
     const ThermoT<double, FAST> T{consts, s_estbl};
     const Column<R, double, ZW, FAST> c(args, T, col, slot);
-    c.template run_body<SPLIT, PART>();
-}
-
-// The whole column pass in one kernel, with all 512 registers of a lane: for calls
-// without list storage (the allocation-free entry point).
-template <class R, bool ZW = false, bool FAST = false>
-__global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1)))
-void forward_kernel(FwdArgs args, int n, const uwshcu_consts* __restrict__ consts, const double* __restrict__ estbl) {
-    forward_body<R, ZW, false, FAST>(args, n, consts, estbl);
+    c.template run_body<true, PART>();
 }
 
 // One part (PART_*) of a split launch, with OCC wavefronts per SIMD as its register budget.
@@ -57,7 +49,89 @@ template <class R, bool ZW, bool FAST, int PART, int OCC>
 __global__ __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(OCC)))
 void forward_kernel_part(FwdArgs args, int n, const uwshcu_consts* __restrict__ consts,
                          const double* __restrict__ estbl) {
-    forward_body<R, ZW, true, FAST, PART>(args, n, consts, estbl);
+    forward_body<R, ZW, FAST, PART>(args, n, consts, estbl);
+}
+
+// S11 of the listed columns (uwshcu_sort.h).  A lane runs one level of its column at a time
+// and takes the next column from the list when its own has ended, so that it does not wait
+// for its wavefront's deepest column: at 1 036 800 x 35 x 3 the wavefronts issue 30 % fewer
+// FP64 instructions, with 0.57 of their lanes active instead of 0.39.  Lanes at levels of
+// their own read scattered addresses, though: from level-major arrays the sorting moved
+// 47 GB and took as long as before (13.4 ms); from records it takes 9.1 ms (11.6 instead
+// of 15.3 at 200003 x 72 x 10).
+//
+// The wavefronts of the grid take the list in pieces of 64 from a queue (queue, 0 at the
+// launch), so a wavefront's columns stay near each other in memory.  Lanes whose column
+// has reached its cloud top wait until kSortReady of them have (or none has a level left):
+// a cloud-top stage and a start cost a wavefront a quarter of a level, however few
+// lanes take them (waiting for 1, 6, 12 and 24 measured 13.4, 13.6, 13.8 and 13.6 ms without records).
+constexpr int kSortReady = 6;
+template <class R, bool ZW, bool FAST, int OCC>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OCC)))
+void sort_kernel(FwdArgs args, int n, int second_pass, int* queue, const uwshcu_consts* __restrict__ consts,
+                 const double* __restrict__ estbl) {
+    __shared__ double s_estbl[UWSHCU_ESTBL_LEN];
+    const int total = valid_items(args, n);
+    if ((int)blockIdx.x * 64 >= total) return;     // fewer pieces than wavefronts
+    // a list that the wavefronts hold at once runs in step: a lane that has ended an
+    // iteration waits for the others
+    const int ready = total > (int)gridDim.x * 64 ? kSortReady : 64;
+    for (int t = threadIdx.x; t < UWSHCU_ESTBL_LEN; t += blockDim.x) s_estbl[t] = estbl[t];
+    __syncthreads();
+    const int lane = threadIdx.x;
+    const ThermoT<double, FAST> T{consts, s_estbl};
+    using Col = Column<R, double, ZW, FAST>;
+    SortState<R, double> q;
+    int slot = 0, col = 0;
+    bool busy = false, ended = false;     // holds a column; its iteration has reached the cloud top
+    int base = 0, left = 0;               // the piece in hand
+    bool dry = false;                     // the queue is empty
+    for (;;) {
+        const int waiting = __popcll(__ballot(busy ? ended : !(dry && left == 0)));
+        if (waiting >= ready || __ballot(busy && !ended) == 0ull) {
+            bool start = false;
+            if (busy && ended) {
+                const Col c(args, T, col, slot);
+                if (q.exit_code == EX_NONE) c.sort_top(q);
+                if (q.exit_code != EX_NONE || q.iter == 3) {
+                    c.sort_store(q, second_pass != 0);
+                    busy = false;
+                } else {
+                    start = true;
+                }
+                ended = false;
+            }
+            for (;;) {
+                const unsigned long long need = __ballot(!busy);
+                if (need == 0ull) break;
+                if (left == 0) {
+                    if (dry) break;
+                    int b = 0;
+                    if (lane == 0) b = atomicAdd(queue, 64);
+                    base = __builtin_amdgcn_readfirstlane(b);
+                    left = total - base < 64 ? total - base : 64;
+                    if (left <= 0) {
+                        left = 0;
+                        dry = true;
+                        break;
+                    }
+                }
+                const int pos = __popcll(need & ((1ull << lane) - 1ull));
+                if (!busy && pos < left) {
+                    item_column(args, base + pos, slot, col);
+                    Col(args, T, col, slot).sort_load(q);
+                    q.iter = 0;
+                    busy = start = true;
+                }
+                const int took = __popcll(need) < left ? __popcll(need) : left;
+                base += took;
+                left -= took;
+            }
+            if (start) Col(args, T, col, slot).sort_begin(q, q.iter + 1);
+            if (__ballot(busy) == 0ull) break;
+        }
+        if (busy && !ended) ended = !Col(args, T, col, slot).sort_level(q);
+    }
 }
 
 // S12-S21 of the listed columns: a workgroup takes 64 of them, wavefront w the levels
@@ -97,41 +171,78 @@ void rest_kernel(FwdArgs args, int n, int final_pass, const uwshcu_consts* __res
     c.rest_team(team, j < nvalid, final_pass != 0);
 }
 
-// Level-parallel set-up: thread t of the launch handles workspace slot t % n and
-// level t / n (+1 for stages 2-4), so that a wavefront covers consecutive columns.
-// Stages 1 and 2: the set-A environment and the wet bulb, before the column pass.
-// Stages 3 and 4: a listed column's set-B environment (S22) after the first pass of a
-// split launch, in the column's own slot, where it continues.  Stage 1 also clears the
-// launch's marks.
+// Level-parallel set-up.  A workgroup handles a tile of 64 consecutive work items and
+// kSetupLevels levels, a wavefront one level of them.  The tiles of one set of columns
+// follow each other on one XCD (workgroups go to the eight in turn), so that the levels
+// below and above, which stage 2 and 4 read as well, are still in its L2: with a level's
+// rows over all columns first, they were read again from HBM.
+// Stages 1 and 2: the set-A environment and the wet bulb, before the column pass; stage 1
+// clears the launch's marks, stage 2 writes the buoyancy sorting's records, through LDS so
+// that whole cache lines go out.  Stages 3 and 4: a listed column's set-B environment (S22)
+// after the first pass of a split launch, in the column's own slot, where it continues.
+constexpr int kSetupLevels = 4;
+__host__ __device__ inline int setup_groups(int stage, int mkx) {
+    return ((stage == 1 ? mkx + 1 : mkx) + kSetupLevels - 1) / kSetupLevels;
+}
+// workgroups of a stage over n items: whole rounds of the eight XCDs
+inline unsigned setup_blocks(int stage, int n, int mkx) {
+    const long long tiles = ((long long)n + 63) / 64;
+    return (unsigned)((tiles + 7) / 8 * 8 * setup_groups(stage, mkx));
+}
 template <class R, int STAGE, bool ZW = false, bool FAST = false>
-__global__ __launch_bounds__(256) void setup_kernel(FwdArgs args, int n, const uwshcu_consts* __restrict__ consts,
-                                                    const double* __restrict__ estbl) {
+__global__ __launch_bounds__(64 * kSetupLevels) void setup_kernel(FwdArgs args, int n,
+                                                                  const uwshcu_consts* __restrict__ consts,
+                                                                  const double* __restrict__ estbl) {
     __shared__ double s_estbl[UWSHCU_ESTBL_LEN];
     const int nvalid = valid_items(args, n);
-    if (STAGE == 1 && args.defer_mark) {   // all n marks, also of slots past a column map's end
-        const long long t0 = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-        if (t0 < n) args.defer_mark[t0] = 0;
+    const int ng = setup_groups(STAGE, args.mkx), r = blockIdx.x >> 3;
+    const int j0 = ((r / ng) * 8 + (int)(blockIdx.x & 7)) * 64;      // the tile's first item
+    if constexpr (STAGE == 1) {   // all n marks, also of slots past a column map's end
+        const int m = j0 + (int)threadIdx.x;
+        if (args.defer_mark && r % ng == 0 && threadIdx.x < 64 && m < n) args.defer_mark[m] = 0;
     }
-    {   // whole workgroup past the listed columns (in one level row): nothing to do
-        const long long t0 = (long long)blockIdx.x * blockDim.x;
-        const long long j0 = t0 % n;
-        if (j0 >= nvalid && j0 + blockDim.x <= n) return;
-    }
+    if (j0 >= nvalid) return;
     for (int t = threadIdx.x; t < UWSHCU_ESTBL_LEN; t += blockDim.x) s_estbl[t] = estbl[t];
     __syncthreads();
-    const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = (int)(t % n);
-    const int k = (int)(t / n) + (STAGE == 1 ? 0 : 1);
-    if (k > args.mkx || j >= nvalid) return;
+    const int lane = threadIdx.x & 63, j = j0 + lane;
+    const int k0 = (r % ng) * kSetupLevels + (STAGE == 1 ? 0 : 1), k = k0 + (threadIdx.x >> 6);
+    const bool work = k <= args.mkx && j < nvalid;
     int slot, col;
-    item_column(args, j, slot, col);
+    item_column(args, j < nvalid ? j : nvalid - 1, slot, col);
     const ThermoT<double, FAST> T{consts, s_estbl};
     const Column<R, double, ZW, FAST> c(args, T, col, slot);
-    if (STAGE >= 3 && c.rstate(RS_CONT) == 0.0) return;   // it ended in its first pass
-    if (STAGE == 1) c.setup_level1(k);
-    else if (STAGE == 2) c.setup_level2(k);
-    else if (STAGE == 3) c.setup_level_b1(k);
-    else c.setup_level_b2(k);
+    if constexpr (STAGE == 1) {
+        if (!work) return;
+        c.setup_level1(k);
+    } else if constexpr (STAGE == 2) {
+        constexpr int kRow = kSetupLevels * kEnvRecord + 2;   // a column's records; 2: bank spread
+        __shared__ double s_rec[std::is_same<R, double>::value ? 64 * kRow : 1];
+        if (work) {
+            const EnvLevelOf<double> e = c.setup_level2(k);
+            if constexpr (std::is_same<R, double>::value) {
+                const double* const v = reinterpret_cast<const double*>(&e);
+                double* const d = s_rec + lane * kRow + (k - k0) * kEnvRecord;
+#pragma unroll
+                for (int q = 0; q < kEnvRecord; ++q) d[q] = v[q];
+            }
+        }
+        if constexpr (std::is_same<R, double>::value) {
+            __syncthreads();
+            // the tile's slots are consecutive: slot j0 + c, levels k0 .. of a column together
+            typedef double f64x2 __attribute__((ext_vector_type(2)));
+            const int levels = args.mkx - k0 + 1 < kSetupLevels ? args.mkx - k0 + 1 : kSetupLevels;
+            const int pieces = levels * kEnvRecord / 2, ncol = nvalid - j0 < 64 ? nvalid - j0 : 64;
+            for (int p = threadIdx.x; p < ncol * pieces; p += 64 * kSetupLevels) {
+                const int cc = p / pieces, q = p % pieces;
+                const f64x2 x{s_rec[cc * kRow + 2 * q], s_rec[cc * kRow + 2 * q + 1]};
+                *reinterpret_cast<f64x2*>(args.rec + ((size_t)(j0 + cc) * (args.mkx + 1) + k0) * kEnvRecord + 2 * q) = x;
+            }
+        }
+    } else {
+        if (!work || c.rstate(RS_CONT) == 0.0) return;   // it ended in its first pass
+        if (STAGE == 3) c.setup_level_b1(k);
+        else c.setup_level_b2(k);
+    }
 }
 
 // Ordered compaction of marks[0, n) into list (slots, ascending) and *count, in three
@@ -159,7 +270,7 @@ static __global__ __launch_bounds__(256) void mark_block_sum_kernel(const int* m
     block_prefix_256(g < n ? marks[g] : 0, s_wave, total);
     if (threadIdx.x == 0) bsum[blockIdx.x] = total;
 }
-static __global__ __launch_bounds__(1024) void block_sum_scan_kernel(int* bsum, int nb, int* count) {
+static __global__ __launch_bounds__(1024) void block_sum_scan_kernel(int* bsum, int nb, int* count, int* queue) {
     __shared__ int s[1024];
     int carry = 0;
     for (int c0 = 0; c0 < nb; c0 += 1024) {
@@ -177,7 +288,10 @@ static __global__ __launch_bounds__(1024) void block_sum_scan_kernel(int* bsum, 
         carry += s[1023];
         __syncthreads();
     }
-    if (threadIdx.x == 0) *count = carry;
+    if (threadIdx.x == 0) {
+        *count = carry;
+        *queue = 0;
+    }
 }
 static __global__ __launch_bounds__(256) void mark_scatter_kernel(int* marks, int n, const int* boff, int* list) {
     __shared__ int s_wave[4];
@@ -199,17 +313,17 @@ static __global__ __launch_bounds__(256) void mark_scatter_kernel(int* marks, in
 //     column that reaches the cloud-base closure saves its scalars and marks itself,
 //     and the marks are compacted into list 1 in column order;
 //  2. the listed (triggered) columns, packed densely, run the rest of the first pass:
-//     the buoyancy sorting (PART_SORT), the stages from the forcedCu filter through the
+//     the buoyancy sorting (sort_kernel), the stages from the forcedCu filter through the
 //     in-cloud diagnostics and the set-B environment, both level-parallel (rest_kernel,
 //     setup stages 3 and 4), and the implicit-CIN iteration up to its CIN (PART_CIN2),
-//     where a column that convects a second time (a few per cent) saves its scalars and
-//     marks itself for list 2;
-//  3. the columns of list 2 run their second convection pass: PART_SORT and rest_kernel.
+//     where a column that convects a second time (a few per cent) goes on through that
+//     pass's closure, saves its scalars and marks itself for list 2;
+//  3. the columns of list 2 run the rest of their second pass: sort_kernel and rest_kernel.
 // Each column keeps its workspace slot throughout.
 //
-// args0.defer_list / defer_state (nullable: the column pass then runs as one kernel) give
-// the lists' storage: defer_count[0..1]; defer_list[0..defer_list_ints(n)): list 1, list 2,
-// the marks and the compaction's block sums; and NRESUME x wld doubles.
+// args0.defer_list / defer_state give the lists' storage: defer_count[0..1];
+// defer_list[0..defer_list_ints(n)): list 1, list 2, the marks, the compaction's block sums
+// and a queue; and NRESUME x wld doubles.  With FP64 plumes args0.rec holds the records.
 template <class R, bool ZW = false, bool FAST = false>
 hipError_t launch_column_pipeline(const FwdArgs& args0, int n, const uwshcu_consts* dconsts, const double* destbl,
                                   hipStream_t stream) {
@@ -222,39 +336,36 @@ hipError_t launch_column_pipeline(const FwdArgs& args0, int n, const uwshcu_cons
     args.list_count = nullptr;
     args.slot0 = args0.col0;
     args.defer_at_closure = 0;
-    const bool split = args0.defer_list && args0.defer_count && args0.defer_state;
+    if (!args0.defer_list || !args0.defer_count || !args0.defer_state || (sizeof(R) == sizeof(double) && !args0.rec))
+        return hipErrorInvalidValue;
     int* const list1 = args0.defer_list;
-    int* const list2 = split ? list1 + (size_t)n : nullptr;
-    int* const marks = split ? list1 + 2 * (size_t)n : nullptr;
-    int* const bsum = split ? list1 + 3 * (size_t)n : nullptr;
+    int* const list2 = list1 + (size_t)n;
+    int* const marks = list1 + 2 * (size_t)n;
+    int* const bsum = list1 + 3 * (size_t)n;
+    int* const queue = bsum + (n + 255) / 256;   // sort_kernel's, cleared by the compaction
     int* const count1 = args0.defer_count;
-    int* const count2 = split ? count1 + 1 : nullptr;
+    int* const count2 = count1 + 1;
     args.defer_mark = marks;
 
-    const unsigned lvl0 = (unsigned)(((long long)n * (args.mkx + 1) + 255) / 256);
-    const unsigned lvl1 = (unsigned)(((long long)n * args.mkx + 255) / 256);
     const dim3 cols((n + 127) / 128), tiles((n + 63) / 64);
-    hipLaunchKernelGGL((setup_kernel<R, 1, ZW, FAST>), dim3(lvl0), dim3(256), 0, stream, args, n, dconsts, destbl);
-    hipLaunchKernelGGL((setup_kernel<R, 2, ZW, FAST>), dim3(lvl1), dim3(256), 0, stream, args, n, dconsts, destbl);
-    if (!split) {
-        hipLaunchKernelGGL((forward_kernel<R, ZW, FAST>), cols, dim3(128), 0, stream, args, n, dconsts, destbl);
-        return hipGetLastError();
-    }
+    hipLaunchKernelGGL((setup_kernel<R, 1, ZW, FAST>), dim3(setup_blocks(1, n, args.mkx)), dim3(64 * kSetupLevels), 0, stream, args, n, dconsts, destbl);
+    hipLaunchKernelGGL((setup_kernel<R, 2, ZW, FAST>), dim3(setup_blocks(2, n, args.mkx)), dim3(64 * kSetupLevels), 0, stream, args, n, dconsts, destbl);
     const unsigned nblk = (unsigned)((n + 255) / 256);
     auto compact = [&](int* list, int* count) {   // marks -> list in column order
         hipLaunchKernelGGL(mark_block_sum_kernel, dim3(nblk), dim3(256), 0, stream, (const int*)marks, n, bsum);
-        hipLaunchKernelGGL(block_sum_scan_kernel, dim3(1), dim3(1024), 0, stream, bsum, (int)nblk, count);
+        hipLaunchKernelGGL(block_sum_scan_kernel, dim3(1), dim3(1024), 0, stream, bsum, (int)nblk, count, queue);
         hipLaunchKernelGGL(mark_scatter_kernel, dim3(nblk), dim3(256), 0, stream, marks, n, (const int*)bsum, list);
     };
     // The buoyancy sorting at two wavefronts per SIMD (256 registers, some spill) where a
     // launch has that many, else at one with all 512.
     const bool large = n >= 2 * 1024 * 64;
-    auto sort = [&](const FwdArgs& f, bool two) {
+    auto sort = [&](const FwdArgs& f, int second_pass, bool two) {
+        const unsigned most = two ? 2048u : 1024u, waves = tiles.x < most ? tiles.x : most;
         if (two)
-            hipLaunchKernelGGL((forward_kernel_part<R, ZW, FAST, PART_SORT, 2>), cols, dim3(128), 0, stream, f, n,
+            hipLaunchKernelGGL((sort_kernel<R, ZW, FAST, 2>), dim3(waves), dim3(64), 0, stream, f, n, second_pass, queue,
                                dconsts, destbl);
         else
-            hipLaunchKernelGGL((forward_kernel_part<R, ZW, FAST, PART_SORT, 1>), cols, dim3(128), 0, stream, f, n,
+            hipLaunchKernelGGL((sort_kernel<R, ZW, FAST, 1>), dim3(waves), dim3(64), 0, stream, f, n, second_pass, queue,
                                dconsts, destbl);
     };
     auto rest = [&](const FwdArgs& f, int final_pass) {
@@ -268,11 +379,10 @@ hipError_t launch_column_pipeline(const FwdArgs& args0, int n, const uwshcu_cons
     b.defer_mark = nullptr;
     b.list = list1;
     b.list_count = count1;
-    b.resume = 1;
-    sort(b, large);
+    sort(b, 0, large);
     rest(b, 0);
-    hipLaunchKernelGGL((setup_kernel<R, 3, ZW, FAST>), dim3(lvl1), dim3(256), 0, stream, b, n, dconsts, destbl);
-    hipLaunchKernelGGL((setup_kernel<R, 4, ZW, FAST>), dim3(lvl1), dim3(256), 0, stream, b, n, dconsts, destbl);
+    hipLaunchKernelGGL((setup_kernel<R, 3, ZW, FAST>), dim3(setup_blocks(3, n, args.mkx)), dim3(64 * kSetupLevels), 0, stream, b, n, dconsts, destbl);
+    hipLaunchKernelGGL((setup_kernel<R, 4, ZW, FAST>), dim3(setup_blocks(4, n, args.mkx)), dim3(64 * kSetupLevels), 0, stream, b, n, dconsts, destbl);
     b.resume = 4;
     b.defer_mark = marks;
     hipLaunchKernelGGL((forward_kernel_part<R, ZW, FAST, PART_CIN2, 2>), cols, dim3(128), 0, stream, b, n, dconsts,
@@ -280,9 +390,8 @@ hipError_t launch_column_pipeline(const FwdArgs& args0, int n, const uwshcu_cons
     compact(list2, count2);
     b.list = list2;
     b.list_count = count2;
-    b.resume = 2;
     b.defer_mark = nullptr;
-    sort(b, false);
+    sort(b, 1, false);
     rest(b, 1);
     return hipGetLastError();
 }

@@ -63,6 +63,8 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
     int kinv = 0, krel = 0, kbup = 0, kpen = -1;
     R prel = 0, cbmf = 0, ufrclcl = 0, ppen = 0, thlu_top = 0, qtu_top = 0;
     D qtsrc = 0, thlsrc = 0, usrc = 0, vsrc = 0;
+    int kwu = 0;                  // the highest level with a velocity
+    R thlu_rel = 0, qtu_rel = 0, wrel = 0, winv = 0;
     int code = EX_NONE;
     live = live && rstate(RS_CONT) != 0.0;
     if (live) {
@@ -70,15 +72,35 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
         prel = R(rstate(13)); cbmf = R(rstate(15)); ufrclcl = R(rstate(17)); ppen = R(rstate(18));
         thlu_top = R(rstate(19)); qtu_top = R(rstate(20));
         kinv = (int)rstate(30); krel = (int)rstate(33); kbup = (int)rstate(34); kpen = (int)rstate(35);
+        thlu_rel = R(rstate(21)); qtu_rel = R(rstate(22)); wrel = R(rstate(26)); winv = R(rstate(28));
+        kwu = (int)rstate(29) > krel - 1 ? (int)rstate(29) : krel - 1;
         amb = (int)rstate(39);
         if (kbup == krel) code = EX_CUFILTER;   // ---- S12 forcedCu filter (uwshcu.F90:2964-2992) ----
     }
     bool run = live && code == EX_NONE;
+    // umf(k) of this pass (uwshcu.F90:2964-2992 clears it from the cloud top up)
+    auto umf_at = [&](int k) -> R {
+        if constexpr (kRec) {
+            if (k >= kpen || k < kinv - 1) return R(0);
+            return k < krel ? cbmf : P(P_UMF, k);
+        } else {
+            return R(out(a.umf, k));
+        }
+    };
     int limit_emf = 0;
 
     if (run) {
-        for (int k = w; k <= mkx; k += nw)
-            if (k >= kpen) out(a.umf, k) = 0.0;
+        for (int k = w; k <= mkx; k += nw) {
+            if constexpr (kRec) {
+                out(a.umf, k) = D(umf_at(k));
+                out(a.wu, k) = k < kinv - 1 || k > kwu ? D(0.0)
+                             : k < krel - 1            ? D(winv)
+                             : k == krel - 1           ? D(wrel)
+                                                       : D(P(P_WU, k));
+            } else {
+                if (k >= kpen) out(a.umf, k) = 0.0;
+            }
+        }
 
         // ---- S13 penetrative entrainment (uwshcu.F90:3055-3183) ----
         if (lead) {
@@ -86,10 +108,10 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
             R emf1 = 0, thlue1 = 0, qtue1 = 0, uue1 = 0, vue1 = 0;   // level k + 1
             for (int k = kpen - 1; k >= kbup; --k) {
                 const R rhos0j = R(in(a.ps0, k)) / (r * R(0.5) * (Er(A_THV0BOT, k + 1) + Er(A_THV0TOP, k)) * Er(A_EXNS0, k));
-                const R umfk = R(out(a.umf, k));
+                const R umfk = umf_at(k);
                 R emfk, thluek, qtuek, uuek, vuek;
                 if (k == kpen - 1) {
-                    const R x = umfk * ppen * W(W_REI, kpen) * rpen;
+                    const R x = umfk * ppen * P(W_REI, kpen) * rpen;
                     const R lim2 = R(-0.9) * R(in(a.dp0, kpen)) / g / dt;
                     if (x < R(-0.1) * rhos0j) limit_emf = 1;
                     if (x < lim2) limit_emf = 1;
@@ -102,7 +124,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                     for (int m = 1; m <= ncnst; ++m)
                             if (tr_entrained(m)) WT(2, m, k) = R(trin(m, kpen)) + WT(0, m, kpen) * dpk;
                 } else {
-                    const R x = emf1 - umfk * R(in(a.dp0, k + 1)) * W(W_REI, k + 1) * rpen;
+                    const R x = emf1 - umfk * R(in(a.dp0, k + 1)) * P(W_REI, k + 1) * rpen;
                     const R lim2 = R(-0.9) * R(in(a.dp0, k + 1)) / g / dt;
                     if (x < R(-0.1) * rhos0j) limit_emf = 1;
                     if (x < lim2) limit_emf = 1;
@@ -197,11 +219,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                 for (int m = kTrLimited; m <= ncnst; ++m)
                     if (tr_moved(m)) WT(3, m, k) = cbmf * (R(trin(m, 1)) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
             } else {
-                const R umfk = R(out(a.umf, k));
-                out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * umfk * (W(W_THLU, k) - (Er(A_THL0, kp1) + Er(A_SSTHL0, kp1) * d)));
-                out(a.qtflx, k) = D(umfk * (W(W_QTU, k) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
-                W(W_UFLX, k) = umfk * (W(W_UU, k) - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
-                W(W_VFLX, k) = umfk * (W(W_VU, k) - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
+                const R umfk = umf_at(k);
+                out(a.slflx, k) = D(cp * Er(A_EXNS0, k) * umfk * (P(W_THLU, k) - (Er(A_THL0, kp1) + Er(A_SSTHL0, kp1) * d)));
+                out(a.qtflx, k) = D(umfk * (P(W_QTU, k) - (Er(A_QT0, kp1) + Er(A_SSQT0, kp1) * d)));
+                W(W_UFLX, k) = umfk * (P(W_UU, k) - (R(in(a.u0, kp1)) + Er(A_SSU0, kp1) * d));
+                W(W_VFLX, k) = umfk * (P(W_VU, k) - (R(in(a.v0, kp1)) + Er(A_SSV0, kp1) * d));
                 for (int m = kTrLimited; m <= ncnst; ++m)
                     if (tr_moved(m)) WT(3, m, k) = umfk * (WT(1, m, k) - (R(trin(m, kp1)) + WT(0, m, kp1) * d));
             }
@@ -213,15 +235,15 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
             D th, qvj, qlj, qij;
             int bad;
             if (k == krel) {
-                if (T.conden(prel, W(W_THLU, krel - 1), W(W_QTU, krel - 1), th, qvj, qlj, qij))
+                if (T.conden(prel, thlu_rel, qtu_rel, th, qvj, qlj, qij))
                     tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
                 W(W_QLR, krel - 1) = R(qlj);
                 W(W_QIR, krel - 1) = R(qij);
-                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij);
+                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
             } else if (k == kpen) {
                 bad = T.conden(R(in(a.ps0, k - 1)) + ppen, thlu_top, qtu_top, th, qvj, qlj, qij);
             } else {
-                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij);
+                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
             }
             if (bad) tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
             W(W_QLR, k) = R(qlj);
@@ -273,7 +295,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
         auto uemf = [&](int k) -> R {   // uwshcu.F90:3416-3422
             if (k <= kinv - 2) return cbmf * (ps00 - R(in(a.ps0, k))) / (ps00 - psinv);
             if (k <= krel - 1) return cbmf;
-            if (k <= kbup - 1) return R(out(a.umf, k));
+            if (k <= kbup - 1) return umf_at(k);
             if (k <= kpen - 1) return W(W_EMF, k);
             return R(0);
         };
@@ -319,10 +341,10 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
 
             const int km1 = k - 1;
             const R dp0k = R(in(a.dp0, k));
-            const R umf_km1 = R(out(a.umf, k - 1)), umf_k = R(out(a.umf, k));
+            const R umf_km1 = umf_at(k - 1), umf_k = umf_at(k);
             // below the release layer the plume arrays hold nothing of this column's plume
-            const R dwk = (k < krel ? R(0) : W(W_DWTEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
-            const R dik = (k < krel ? R(0) : W(W_DITEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
+            const R dwk = (k < krel ? R(0) : P(W_DWTEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
+            const R dik = (k < krel ? R(0) : P(W_DITEN, k)) * R(0.5) * (umf_km1 + umf_k) * g / dp0k;
             const R qrk = frc_rasn * dwk, qsk = frc_rasn * dik;
             out(a.qrten, k) = D(qrk);
             out(a.qsten, k) = D(qsk);
@@ -366,7 +388,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
             R qc_i = (R(1) - frc_rasn) * dik;
             R qc_lm, qc_im, nc_lm, nc_im;
             if (k <= kbup) {
-                const R fdrk = k < krel ? R(0) : W(W_FDR, k);
+                const R fdrk = k < krel ? R(0) : P(W_FDR, k);
                 qc_l = qc_l + g * R(0.5) * (umf_km1 + umf_k) * fdrk * qlu_mid;
                 qc_i = qc_i + g * R(0.5) * (umf_km1 + umf_k) * fdrk * qiu_mid;
                 qc_lm = -g * R(0.5) * (umf_km1 + umf_k) * fdrk * ql0k;
@@ -555,23 +577,23 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                     R tmp1 = (R(in(a.z0, k)) - R(in(a.z0, krel))) / (R(in(a.z0, kpen)) - R(in(a.z0, krel)) + R(10));
                     tmp1 = R(1) + R(a.zw.ufrcz) * tmp1;
                     tmp3 = tmp3 * tmp1;
-                    tmp2 = W(W_FDR, k) * R(out(a.umf, k)) * R(in(a.zs0, k) - in(a.zs0, k - 1)) * dt /
+                    tmp2 = P(W_FDR, k) * umf_at(k) * R(in(a.zs0, k) - in(a.zs0, k - 1)) * dt /
                            R(in(a.dp0, k)) * R(9.8) * R(a.zw.ufrcd);
                     tmp2 = fmin(R(1) - rmaxfrac, tmp2);
                 }
             }
             R cufrck;
             if (k == krel) {
-                cufrck = (ufrclcl + W(W_UFRC, k)) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                cufrck = (ufrclcl + P(W_UFRC, k)) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
             } else if (k == kpen) {
-                cufrck = (W(W_UFRC, k - 1) + R(0)) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
+                cufrck = (P(W_UFRC, k - 1) + R(0)) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
                 if ((qlr + qir) > criqc) {
                     qcuk = R(0.5) * (qcubelow + criqc);
                     qluk = R(0.5) * (qlubelow + criqc * qlr / (qlr + qir));
                     qiuk = R(0.5) * (qiubelow + criqc * qir / (qlr + qir));
                 }
             } else {
-                cufrck = (W(W_UFRC, k - 1) + W(W_UFRC, k));
+                cufrck = (P(W_UFRC, k - 1) + P(W_UFRC, k));
             }
             out(a.qcu, k) = D(qcuk);
             out(a.qlu, k) = D(qluk);

@@ -105,7 +105,8 @@ int uwshcu_forward_device(uwshcu_ctx *ctx, int precision, const uwshcu_params *p
 /* uwshcu_forward_device(ctx, UWSHCU_FP64, ...) for callers that cannot allocate device
  * memory: code under HIP graph capture, tight serving loops, harnesses that forbid
  * hipMalloc.  No counterpart in the reference.  The call allocates nothing: its
- * workspace is a static device array of UWSHCU_NOALLOC_SCRATCH_BYTES (256 MiB) per GPU,
+ * workspace is a static device array of UWSHCU_NOALLOC_SCRATCH_BYTES (256 MiB) per GPU
+ * (and, since its launch is split by stage, 161 MiB for the lists of its columns),
  * whose address uwshcu_ctx_create looks up.  The chunk needs
  * uwshcu_workspace_bytes_per_column(pver, ncnst, UWSHCU_FP64) bytes for each of its ncol
  * columns rounded up to a multiple of 64 (at 35 levels and 3 constituents up to 14 528
