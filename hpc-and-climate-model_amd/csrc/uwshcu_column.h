@@ -47,7 +47,9 @@ enum EnvArray : int {
     B_THL0, B_QT0, B_SSTHL0, B_SSQT0, B_THV0BOT, B_THV0TOP, B_THVL0BOT, B_THVL0TOP,
     E_QVSTAR,
     E_THV0MID, E_QS0MID,   // saturation state of the layer-mean environment, filled when first used
-    ENV_ARRAYS
+    ENV_ARRAYS,
+    // S19's terms of a pass (rest_team), in arrays that are free then: set B is formed later
+    E_DQL = B_THL0, E_DQI = B_QT0, E_QVTEN = B_SSTHL0
 };
 // Plume and flux working arrays, in the bulk type R.
 enum WsArray : int {
@@ -577,6 +579,11 @@ struct Column {
             out(a.sten, k) = sten;
             E(E_QVSTAR, k) = qv;
         }
+        spread_moisture(dqv);
+    }
+    // the lowest layer's lack, taken from all layers that have vapour to give
+    UWSHCU_HD UW_INLINE void spread_moisture(D dqv) const {
+        const double dtd = a.dt, qvmin = C.qmin[1];
         if (dqv > 1.e-20) {
             D sum = 0.0;
             for (int k = 1; k <= mkx; ++k) {

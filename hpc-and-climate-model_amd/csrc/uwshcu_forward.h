@@ -135,13 +135,17 @@ void sort_kernel(FwdArgs args, int n, int second_pass, int* queue, const uwshcu_
 }
 
 // S12-S21 of the listed columns: a workgroup takes 64 of them, wavefront w the levels
-// w, w + kRestWaves, ... (uwshcu_rest.h).
-constexpr int kRestWaves = 8;
+// w, w + kRestWaves, ... (uwshcu_rest.h).  Bound by memory: it waits for loads and stores of
+// 34 GB at 1 036 800 x 35 x 3.  Four wavefronts, two workgroups on a CU: both passes take
+// 11.0 ms there, with eight 12.2; with four the stages that one wavefront runs
+// alone leave fewer idle.  The fast path's saturation adjustment takes more registers than
+// two workgroups leave; held to them (with spills) its two passes take 7.9 ms, else 9.5.
+constexpr int kRestWaves = 4;
 struct TileTeam {
     int rank;
     static constexpr int size = kRestWaves;
     int* s_fail;      // [64] smallest failure of each column
-    int* s_borrow;    // [64]
+    int* s_borrow;     // [64]
     __device__ void sync() { __syncthreads(); }
     __device__ void fail(int key) { atomicMin(&s_fail[threadIdx.x & 63], key); }
     __device__ int failed() const { return s_fail[threadIdx.x & 63]; }
@@ -149,7 +153,7 @@ struct TileTeam {
     __device__ bool borrowed() const { return s_borrow[threadIdx.x & 63] != 0; }
 };
 template <class R, bool ZW, bool FAST>
-__global__ __launch_bounds__(64 * kRestWaves)
+__global__ __launch_bounds__(64 * kRestWaves) __attribute__((amdgpu_waves_per_eu(FAST ? 2 : 1)))
 void rest_kernel(FwdArgs args, int n, int final_pass, const uwshcu_consts* __restrict__ consts,
                  const double* __restrict__ estbl) {
     __shared__ double s_estbl[UWSHCU_ESTBL_LEN];

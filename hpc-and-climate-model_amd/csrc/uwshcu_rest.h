@@ -12,7 +12,11 @@
 // 1 036 800 x 35 x 3, most of a small launch's second half).  Here a workgroup takes 64
 // columns of the list and its wavefronts the levels in turn, so a column has as many
 // accesses in flight as there are wavefronts, and a wavefront's accesses stay one
-// 64-column row per array and level: 9.9 ms there, 35 GB moved; 0.4 ms at 32768 columns.
+// 64-column row per array and level.  The sequential parts hold up a whole tile, so they
+// keep only the recurrence: the condensate raise (S19) is done where a level's tendencies
+// are formed, and column by column only where the vapour lacks (2 % of them), and S17
+// reads a level ahead and stores the final tendencies.  Both passes take 11.0 ms there
+// (12.3 with S18 and S19 as steps of their own); 0.61 ms at 32768 columns.
 //
 // The same code runs on the host with a team of one (every stage over all levels in
 // turn).  Each value is computed by the sequential stages' operations in their order, so
@@ -26,13 +30,14 @@ namespace uwshcu {
 
 // A team of one thread: takes every level.
 struct SerialTeam {
-    int fail_key = 0x7fffffff, borrow = 0;
+    int fail_key = 0x7fffffff;
+    bool borrow = false;
     static constexpr int rank = 0, size = 1;
     UWSHCU_HD void sync() {}
     UWSHCU_HD void fail(int key) { fail_key = key < fail_key ? key : fail_key; }
     UWSHCU_HD int failed() const { return fail_key; }
-    UWSHCU_HD void borrows() { borrow = 1; }
-    UWSHCU_HD bool borrowed() const { return borrow != 0; }
+    UWSHCU_HD void borrows() { borrow = true; }
+    UWSHCU_HD bool borrowed() const { return borrow; }
 };
 
 // live: this thread's column takes part (every thread of a team calls this, for the
@@ -290,6 +295,20 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
     tm.sync();
 
     // ---- S15 subsidence condensate sinks, S16 tendencies (uwshcu.F90:3416-3794) ----
+    // S19 (positive_moisture) raises a layer's condensate to its minimum from the layer's own
+    // vapour; only where the vapour then lacks does it borrow from the layer below.  The
+    // first is done where a level's tendencies are formed, the second column by column.
+    const double qvmin = C.qmin[1], qlmin = C.qmin[2], qimin = C.qmin[3];
+    const double xlvd = C.xlv, xlsd = C.xls;
+    auto raise_water = [&](int k, D qlten, D qiten) {   // stores both, and what was added
+        const D ql = in(a.ql0, k) + qlten * dtd, qi = in(a.qi0, k) + qiten * dtd;
+        const D dql = fmax(0.0, 1.0 * qlmin - ql), dqi = fmax(0.0, 1.0 * qimin - qi);
+        out(a.qlten, k) = qlten + dql / dtd;
+        out(a.qiten, k) = qiten + dqi / dtd;
+        E(E_DQL, k) = dql;
+        E(E_DQI, k) = dqi;
+    };
+    auto lacks = [&](D qv0, D qvten, D dql, D dqi) { return 1.0 * qvmin - (qv0 + qvten * dtd - dql - dqi) > 0.0; };
     if (run) {
         const R ps00 = R(in(a.ps0, 0)), psinv = R(in(a.ps0, kinv - 1));
         auto uemf = [&](int k) -> R {   // uwshcu.F90:3416-3422
@@ -301,8 +320,22 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
         };
         auto uf = [&](int k) -> R { return R(in(a.u0, k)) + R(out(a.uten, k)) * dt; };
         auto vf = [&](int k) -> R { return R(in(a.v0, k)) + R(out(a.vten, k)) * dt; };
-        for (int k = w; k <= kpen; k += nw) {
+        for (int k = w; k <= mkx; k += nw) {
             if (k < 1) continue;
+            if (k > kpen) {   // above the cloud: every store of this loop, so that lines go out whole
+                out(a.qrten, k) = 0.0;
+                out(a.qsten, k) = 0.0;
+                out(a.qc, k) = 0.0;
+                out(a.evapc, k) = 0.0;
+                if (has_nl) trout(ixl, k) = 0.0;
+                if (has_ni) trout(ixi, k) = 0.0;
+                raise_water(k, 0.0, 0.0);
+                const D dql = E(E_DQL, k), dqi = E(E_DQI, k);
+                out(a.qvten, k) = 0.0 - (dql + dqi) / dtd;
+                out(a.sten, k) = 0.0 + xlvd * (dql / dtd) + xlsd * (dqi / dtd);
+                if (lacks(in_qv0(k), 0.0, dql, dqi)) tm.borrows();
+                continue;
+            }
             D th, qvj, qlj, qij;
             const R comsub = R(0.5) * (uemf(k) + uemf(k - 1));
             const R thl0k = Er(A_THL0, k), qt0k = Er(A_QT0, k), ql0k = R(in(a.ql0, k)), qi0k = R(in(a.qi0, k));
@@ -421,11 +454,10 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
             const R qitenk = qc_i + frc_rasn * dik + (fmax(R(0), qi0k + (qc_im + qisink) * dt) - qi0k) / dt;
             if (has_nl) trout(ixl, k) = D(fmax(nc_lm + nlsink, -trz(ixl, k) / dt));
             if (has_ni) trout(ixi, k) = D(fmax(nc_im + nisink, -trz(ixi, k) / dt));
-            out(a.qlten, k) = D(qltenk);
-            out(a.qiten, k) = D(qitenk);
             out(a.qvten, k) = D(qtten - qltenk - qitenk);
             out(a.sten, k) = D(slten + xlv * qltenk + xls * qitenk);
-            W(W_QCL, k) = qc_l;
+            // S17's and S18's terms of the condensate tendencies (uwshcu.F90:3966-3981)
+            raise_water(k, D(qltenk - qrk - qc_l), D(qitenk - qsk - qc_i));
             W(W_QCI, k) = qc_i;
             out(a.qc, k) = D(qc_l + qc_i);
             // for S17: the evaporation's rate but for the flux, and its limit
@@ -457,22 +489,30 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
         // (above it there is no flux, and every term is zero) ----
         if (lead) {
             R rliq = R(0), rainflx = R(0), snowflx = R(0);
+#pragma unroll 4
             for (int k = 1; k <= kpen; ++k) {
                 const R dp0k = R(in(a.dp0, k));
                 rainflx = rainflx + R(out(a.qrten, k)) * dp0k / g;
                 snowflx = snowflx + R(out(a.qsten, k)) * dp0k / g;
                 rliq = rliq + R(out(a.qc, k)) * dp0k / g / R(1000);
             }
+            // a level's values are read while the one above is computed
+            struct Level { R dp0, rate, limit, qr, qs, qci; D t0, qv0, qvten, sten, dql, dqi; };
+            auto load = [&](int k) {
+                return Level{R(in(a.dp0, k)), W(W_TRFD, k), W(W_TRFU, k), R(out(a.qrten, k)), R(out(a.qsten, k)),
+                             W(W_QCI, k), in_t0(k), in_qv0(k), out(a.qvten, k), out(a.sten, k),
+                             E(E_DQL, k), E(E_DQI, k)};
+            };
             R flxrain_k = R(0), flxsnow_k = R(0);   // fluxes at the top interface of layer k
             R evpint_rain = R(0), evpint_snow = R(0);
+            Level next = load(kpen);
             for (int k = kpen; k >= 1; --k) {
-                const R dp0k = R(in(a.dp0, k));
-                const R t0k = R(in_t0(k));
-                const R rate = W(W_TRFD, k), evplimit = W(W_TRFU, k);
-                const R qrk = R(out(a.qrten, k)), qsk = R(out(a.qsten, k));
+                const Level v = next;
+                next = load(k > 1 ? k - 1 : 1);
+                const R dp0k = v.dp0, t0k = R(v.t0), evplimit = v.limit;
                 R snowmlt = (t0k > R(273.16)) ? fmax(R(0), flxsnow_k * g / dp0k) : R(0);
-                R evprain = rate * sqrt(flxrain_k + snowmlt * dp0k / g);
-                R evpsnow = rate * sqrt(fmax(flxsnow_k - snowmlt * dp0k / g, R(0)));
+                R evprain = v.rate * sqrt(flxrain_k + snowmlt * dp0k / g);
+                R evpsnow = v.rate * sqrt(fmax(flxsnow_k - snowmlt * dp0k / g, R(0)));
                 R evplimit_rain = fmin(evplimit, (flxrain_k + snowmlt * dp0k / g) * g / dp0k);
                 evplimit_rain = fmin(evplimit_rain, (rainflx - evpint_rain) * g / dp0k);
                 evprain = fmax(R(0), fmin(evplimit_rain, evprain));
@@ -487,17 +527,24 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                 }
                 evpint_rain = evpint_rain + evprain * dp0k / g;
                 evpint_snow = evpint_snow + evpsnow * dp0k / g;
-                const R ntraprd = qrk - evprain + snowmlt;
-                const R ntsnprd = qsk - evpsnow - snowmlt;
+                const R ntraprd = v.qr - evprain + snowmlt;
+                const R ntsnprd = v.qs - evpsnow - snowmlt;
                 const R flxrain_km1 = fmax(flxrain_k + ntraprd * dp0k / g, R(0));
                 const R flxsnow_km1 = fmax(flxsnow_k + ntsnprd * dp0k / g, R(0));
                 flxrain_k = flxrain_km1;
                 flxsnow_k = flxsnow_km1;
-                out(a.flxprc1, k - 1) = final_pass ? D(flxrain_km1 + flxsnow_km1) : D(0.0);
-                out(a.flxsnow1, k - 1) = final_pass ? D(flxsnow_km1) : D(0.0);
-                W(W_QLSINK, k) = evprain;
-                W(W_QISINK, k) = evpsnow;
-                W(W_NLSINK, k) = snowmlt;
+                if (final_pass) {
+                    out(a.flxprc1, k - 1) = D(flxrain_km1 + flxsnow_km1);
+                    out(a.flxsnow1, k - 1) = D(flxsnow_km1);
+                }
+                // the tendencies, with S18's reserved ice
+                const D qvten = D(R(v.qvten) + evprain + evpsnow);
+                const R st = R(v.sten) - xlv * evprain - xls * evpsnow - (xls - xlv) * snowmlt;
+                out(a.evapc, k) = D(evprain + evpsnow);
+                E(E_QVTEN, k) = qvten;
+                out(a.qvten, k) = qvten - (v.dql + v.dqi) / dtd;
+                out(a.sten, k) = D(st - (xls - xlv) * v.qci) + xlvd * (v.dql / dtd) + xlsd * (v.dqi / dtd);
+                if (lacks(v.qv0, qvten, v.dql, v.dqi)) tm.borrows();
             }
             cout(a.precip) = D((flxrain_k + flxsnow_k) / R(1000));
             cout(a.snow) = D(flxsnow_k / R(1000));
@@ -543,18 +590,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
         // ---- S21 in-cloud diagnostics (uwshcu.F90:4092-4158), and the zeros of the levels
         // outside the cloud ----
         for (int k = w; k <= mkx; k += nw) {
-            if (k >= kpen) {
+            if (k >= kpen || !final_pass) {
                 out(a.flxprc1, k) = 0.0;
                 out(a.flxsnow1, k) = 0.0;
             }
             if (k < 1) continue;
-            if (k > kpen) {
-                out(a.qrten, k) = 0.0;
-                out(a.qsten, k) = 0.0;
-                out(a.qc, k) = 0.0;
-                if (has_nl) trout(ixl, k) = 0.0;
-                if (has_ni) trout(ixi, k) = 0.0;
-            }
             for (int m = 1; m <= ncnst && m < kTrLimited; ++m)
                 if (m != ixl && m != ixi) trout(m, k) = 0.0;
             if (k < krel || k > kpen) {
@@ -604,57 +644,31 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
     }
     tm.sync();
 
-    // ---- S17's tendencies, S18 reserved condensate (uwshcu.F90:3966-3981) and S19 positive
-    // moisture, FP64 (uwshcu.F90:3995-4001, 5096-5162) ----
-    const double qvmin = C.qmin[1], qlmin = C.qmin[2], qimin = C.qmin[3];
-    unsigned adjusted = 0;   // this thread's levels (bit (k - w) / nw) that S19 changes
-    if (run) {
-        for (int k = w, bit = 0; k <= mkx; k += nw, ++bit) {
-            if (k < 1) continue;
-            D qvten = 0.0, qlten = 0.0, qiten = 0.0, sten = 0.0;
-            if (k <= kpen) {
-                const R evprain = W(W_QLSINK, k), evpsnow = W(W_QISINK, k), snowmlt = W(W_NLSINK, k);
-                const R qcl = W(W_QCL, k), qci = W(W_QCI, k);
-                out(a.evapc, k) = D(evprain + evpsnow);
-                const R qlt = R(out(a.qlten, k)) - R(out(a.qrten, k));
-                const R qit = R(out(a.qiten, k)) - R(out(a.qsten, k));
-                const R qvt = R(out(a.qvten, k)) + evprain + evpsnow;
-                const R st = R(out(a.sten, k)) - xlv * evprain - xls * evpsnow - (xls - xlv) * snowmlt;
-                qvten = D(qvt);
-                qlten = D(qlt - qcl);
-                qiten = D(qit - qci);
-                sten = D(st - (xls - xlv) * qci);
-            } else {
-                out(a.evapc, k) = 0.0;
+    // ---- S19 where a layer's vapour lacks (uwshcu.F90:3995-4001, 5096-5162) ----
+    if (run && lead && tm.borrowed()) {
+        D dqv = 0.0, carry_qv = 0.0, carry_ten = 0.0;   // taken from layer k-1 for layer k
+        for (int k = mkx; k >= 1; --k) {
+            const D dql = E(E_DQL, k), dqi = E(E_DQI, k);
+            D qvten = k <= kpen ? E(E_QVTEN, k) : D(0.0);
+            D qv = in_qv0(k) + qvten * dtd;
+            if (k != mkx) {
+                qv = qv - carry_qv;
+                qvten = qvten - carry_ten;
+            }
+            qvten = qvten - (dql + dqi) / dtd;
+            qv = qv - dql - dqi;
+            dqv = fmax(0.0, 1.0 * qvmin - qv);
+            qvten = qvten + dqv / dtd;
+            qv = qv + dqv;
+            if (k != 1) {
+                const D dpk = in(a.dp0, k), dpkm1 = in(a.dp0, k - 1);
+                carry_qv = dqv * dpk / dpkm1;
+                carry_ten = dqv * dpk / dpkm1 / dtd;
             }
             out(a.qvten, k) = qvten;
-            out(a.qlten, k) = qlten;
-            out(a.qiten, k) = qiten;
-            out(a.sten, k) = sten;
-            const D ql = in(a.ql0, k) + qlten * dtd, qi = in(a.qi0, k) + qiten * dtd;
-            const D dql = fmax(0.0, 1.0 * qlmin - ql), dqi = fmax(0.0, 1.0 * qimin - qi);
-            const D qv = in_qv0(k) + qvten * dtd - dql - dqi;
-            if (1.0 * qvmin - qv > 0.0) tm.borrows();      // it borrows from the layer below
-            if (dql != 0.0 || dqi != 0.0) adjusted |= 1u << (bit & 31);
+            E(E_QVSTAR, k) = fmax(qv, qvmin);
         }
-    }
-    tm.sync();
-    if (!run) return;
-    const double xlvd = C.xlv, xlsd = C.xls;
-    if (!tm.borrowed()) {
-        // no layer runs dry: each level's own condensate adjustment
-        for (int k = w, bit = 0; k <= mkx; k += nw, ++bit) {
-            if (k < 1 || !(adjusted >> (bit & 31) & 1u)) continue;
-            D qvten = out(a.qvten, k), qlten = out(a.qlten, k), qiten = out(a.qiten, k), sten = out(a.sten, k);
-            const D ql = in(a.ql0, k) + qlten * dtd, qi = in(a.qi0, k) + qiten * dtd;
-            const D dql = fmax(0.0, 1.0 * qlmin - ql), dqi = fmax(0.0, 1.0 * qimin - qi);
-            out(a.qlten, k) = qlten + dql / dtd;
-            out(a.qiten, k) = qiten + dqi / dtd;
-            out(a.qvten, k) = qvten - (dql + dqi) / dtd;
-            out(a.sten, k) = sten + xlvd * (dql / dtd) + xlsd * (dqi / dtd);
-        }
-    } else if (lead) {
-        positive_moisture();
+        spread_moisture(dqv);
     }
 }
 
