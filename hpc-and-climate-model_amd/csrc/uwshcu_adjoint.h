@@ -38,10 +38,11 @@ UWSHCU_HD inline void ad_begin(TapeCtx& t, TapeHot& h, TapeNode* nodes, int* pag
         t.ctr = nullptr;
         t.shard_base = 0;
     }
-    for (int q = 0; q < nin; ++q) {
-        if (q >= h.limit && !tape_grow(t, h, q)) break;
+    if (h.n >= h.limit) tape_grow(t, h);
+    for (int q = 0; q < nin && t.overflow != 1; ++q) {
+        if (h.nodes && q < cap && (!pool || pool->sink || t.overflow == 0)) tape_store(h.nodes - q, 0.0, 0.0, -1, -1);
         h.n = q + 1;
-        if (TapeNode* top = h.nodes) tape_store(top - q, 0.0, 0.0, -1, -1);
+        if (h.n >= h.limit) tape_grow(t, h);
     }
     t.hot = h;
 }

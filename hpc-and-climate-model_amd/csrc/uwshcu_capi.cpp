@@ -373,7 +373,7 @@ int run_adjoint(uwshcu_ctx* ctx, const uwshcu_params* par, int pcols, int ncol, 
         o[3] = o[2] + align256(sizeof(TapeCtx) * nb);
         o[4] = o[3] + align256((size_t)maxp * sizeof(int) * nb);
         o[5] = o[4] + align256(sizeof(TapePool));
-        o[6] = o[5] + align256(sizeof(TapeNode) * kTapePage * npages);
+        o[6] = o[5] + align256(sizeof(TapeNode) * kTapePage * (npages + 1));   // the last page is the sink
         o[7] = o[6] + align256(sizeof(double) * kTapePage * npages);
     };
     double* parcol = grad->par_col;
@@ -466,6 +466,7 @@ int run_adjoint(uwshcu_ctx* ctx, const uwshcu_params* par, int pcols, int ncol, 
         a.ad.tapes = (TapeCtx*)(base + oo[2]);
         std::memset(hp, 0, sizeof(TapePool));
         hp->base = (TapeNode*)(base + oo[5]);
+        hp->sink = hp->base + (size_t)kTapePage * npages;
         hp->nshards = nshards;
         hp->per_shard = (int)(npages / (size_t)nshards);
         TapePool* dpool = (TapePool*)(base + oo[4]);
@@ -513,7 +514,9 @@ int run_adjoint(uwshcu_ctx* ctx, const uwshcu_params* par, int pcols, int ncol, 
             size_t need = 0;
             long long s1 = s0;
             while (s1 < n) {
-                const size_t pc = ((size_t)(hdr[s1].hot.n < cap ? hdr[s1].hot.n : cap) + kTapePage - 1) / kTapePage;
+                // a tape of n nodes has taken the page of its next one
+                const size_t nodes = hdr[s1].hot.n < cap ? (size_t)hdr[s1].hot.n + 1 : (size_t)cap;
+                const size_t pc = (nodes + kTapePage - 1) / kTapePage;
                 if (s1 > s0 && need + pc > room(s1 + 1 - s0)) break;
                 need += pc;
                 ++s1;

@@ -72,6 +72,47 @@ UWSHCU_HD inline size_t ws_bytes_per_column(int mkx, int ncnst, size_t r_size, s
     return (size_t)(mkx + 1) * ((size_t)ENV_ARRAYS * d_size + (size_t)ws_arrays(ncnst) * r_size);
 }
 
+// Reverse-mode state of one launch (adjoint kernel only).  Output fields are held as
+// tape values while the column runs: field f, level k of workspace slot j lives at
+// out[(f * (mkx+1) + k) * wld + j]; fields are ADF_* below, then trten(m) at
+// ADF_TR + m - 1, then the column scalars at ADF_TR + ncnst + ADC_*.
+enum AdField : int {
+    ADF_UMF, ADF_SLFLX, ADF_QTFLX, ADF_FLXPRC1, ADF_FLXSNOW1, ADF_WU,
+    ADF_QVTEN, ADF_QLTEN, ADF_QITEN, ADF_STEN, ADF_UTEN, ADF_VTEN, ADF_QRTEN, ADF_QSTEN, ADF_EVAPC,
+    ADF_CUFRC, ADF_QCU, ADF_QLU, ADF_QIU, ADF_QC,
+    ADF_TR
+};
+enum AdColumnField : int { ADC_PRECIP, ADC_SNOW, ADC_CBMF, ADC_RLIQ, ADC_CNT, ADC_CNB, ADC_CUSH, ADC_COUNT };
+UWSHCU_HD inline int ad_fields(int ncnst) { return ADF_TR + ncnst + ADC_COUNT; }
+// Independent variables: node f*(mkx+1)+k for t0, qv0, u0, v0 (f = 0..3, k = 1..mkx)
+// and tke (f = 4, k = 0..mkx), then rpen, rle, rkm.
+enum AdInput : int { ADI_T0, ADI_QV0, ADI_U0, ADI_V0, ADI_TKE, ADI_PARAMS };
+UWSHCU_HD inline int ad_inputs(int mkx) { return ADI_PARAMS * (mkx + 1) + 3; }
+
+// A caller array that the adjoint follows, with its field known at compile time: an input
+// (AdInput F), an output (AdField F) or a column scalar (AdColumnField F).  The recording then
+// knows at each access which tape entry is meant and that every other input is a constant;
+// from the pointers alone it compared them at every access, and recorded, or tested
+// whether to record, every operation on pressures and heights as well.
+template <int F>
+struct AdIn {
+    const double* p;
+    UWSHCU_HD AdIn& operator=(const double* q) { p = q; return *this; }
+    UWSHCU_HD operator const double*() const { return p; }
+};
+template <int F>
+struct AdOut {
+    double* p;
+    UWSHCU_HD AdOut& operator=(double* q) { p = q; return *this; }
+    UWSHCU_HD operator double*() const { return p; }
+};
+template <int F>
+struct AdScalar {
+    double* p;
+    UWSHCU_HD AdScalar& operator=(double* q) { p = q; return *this; }
+    UWSHCU_HD operator double*() const { return p; }
+};
+
 // Reverse-mode state of one launch (adjoint kernel only; null pointers otherwise).
 struct AdArgs {
     AD* out;           // tape values of the outputs (layout: AdField below)
@@ -84,10 +125,43 @@ struct FwdArgs {
     long long wld;
     double dt;
     uwshcu_params par;
-    const double *ps0, *zs0, *p0, *z0, *dp0, *dpdry0, *u0, *v0, *qv0, *ql0, *qi0, *t0, *s0, *tr0, *tke, *pblh;
-    double* cush;
-    double *umf, *slflx, *qtflx, *flxprc1, *flxsnow1, *qvten, *qlten, *qiten, *sten, *uten, *vten, *trten;
-    double *qrten, *qsten, *precip, *snow, *evapc, *cufrc, *qcu, *qlu, *qiu, *cbmf, *qc, *rliq, *cnt, *cnb, *wu;
+    const double *ps0, *zs0, *p0, *z0, *dp0, *dpdry0;
+    AdIn<ADI_U0> u0;
+    AdIn<ADI_V0> v0;
+    AdIn<ADI_QV0> qv0;
+    const double *ql0, *qi0;
+    AdIn<ADI_T0> t0;
+    const double *s0, *tr0;
+    AdIn<ADI_TKE> tke;
+    const double* pblh;
+    AdScalar<ADC_CUSH> cush;
+    AdOut<ADF_UMF> umf;
+    AdOut<ADF_SLFLX> slflx;
+    AdOut<ADF_QTFLX> qtflx;
+    AdOut<ADF_FLXPRC1> flxprc1;
+    AdOut<ADF_FLXSNOW1> flxsnow1;
+    AdOut<ADF_QVTEN> qvten;
+    AdOut<ADF_QLTEN> qlten;
+    AdOut<ADF_QITEN> qiten;
+    AdOut<ADF_STEN> sten;
+    AdOut<ADF_UTEN> uten;
+    AdOut<ADF_VTEN> vten;
+    double* trten;
+    AdOut<ADF_QRTEN> qrten;
+    AdOut<ADF_QSTEN> qsten;
+    AdScalar<ADC_PRECIP> precip;
+    AdScalar<ADC_SNOW> snow;
+    AdOut<ADF_EVAPC> evapc;
+    AdOut<ADF_CUFRC> cufrc;
+    AdOut<ADF_QCU> qcu;
+    AdOut<ADF_QLU> qlu;
+    AdOut<ADF_QIU> qiu;
+    AdScalar<ADC_CBMF> cbmf;
+    AdOut<ADF_QC> qc;
+    AdScalar<ADC_RLIQ> rliq;
+    AdScalar<ADC_CNT> cnt;
+    AdScalar<ADC_CNB> cnb;
+    AdOut<ADF_WU> wu;
     int* diag;          // optional [UWSHCU_NDIAG][ldc]
     int* err;           // [2]: first fatal code, column
     void* ws;           // workspace (see ws_bytes_per_column)
@@ -135,23 +209,6 @@ UWSHCU_HD inline double zmh_ramp(double x, double x0, double xint) {
     else x2 = (x - x0) / fmax(xint, (double)1.e-20f);
     return fmin(x2, 1.0);
 }
-
-// Reverse-mode state of one launch (adjoint kernel only).  Output fields are held as
-// tape values while the column runs: field f, level k of workspace slot j lives at
-// out[(f * (mkx+1) + k) * wld + j]; fields are ADF_* below, then trten(m) at
-// ADF_TR + m - 1, then the column scalars at ADF_TR + ncnst + ADC_*.
-enum AdField : int {
-    ADF_UMF, ADF_SLFLX, ADF_QTFLX, ADF_FLXPRC1, ADF_FLXSNOW1, ADF_WU,
-    ADF_QVTEN, ADF_QLTEN, ADF_QITEN, ADF_STEN, ADF_UTEN, ADF_VTEN, ADF_QRTEN, ADF_QSTEN, ADF_EVAPC,
-    ADF_CUFRC, ADF_QCU, ADF_QLU, ADF_QIU, ADF_QC,
-    ADF_TR
-};
-enum AdColumnField : int { ADC_PRECIP, ADC_SNOW, ADC_CBMF, ADC_RLIQ, ADC_CNT, ADC_CNB, ADC_CUSH, ADC_COUNT };
-UWSHCU_HD inline int ad_fields(int ncnst) { return ADF_TR + ncnst + ADC_COUNT; }
-// Independent variables: node f*(mkx+1)+k for t0, qv0, u0, v0 (f = 0..3, k = 1..mkx)
-// and tke (f = 4, k = 0..mkx), then rpen, rle, rkm.
-enum AdInput : int { ADI_T0, ADI_QV0, ADI_U0, ADI_V0, ADI_TKE, ADI_PARAMS };
-UWSHCU_HD inline int ad_inputs(int mkx) { return ADI_PARAMS * (mkx + 1) + 3; }
 
 // Exit reasons reported in diag row 0 (same numbering as the oracle).
 // Scalars of a column deferred at its second convection pass (FwdArgs::defer_state).
@@ -285,28 +342,15 @@ struct Column {
         if constexpr (kAD) return a.ad.out[((size_t)f * KS + k) * wld + iw];
         else return *(D*)nullptr;
     }
-    UWSHCU_HD inline int ad_field(const double* p) const {
-        const double* const f[] = {a.umf, a.slflx, a.qtflx, a.flxprc1, a.flxsnow1, a.wu, a.qvten, a.qlten, a.qiten,
-                                   a.sten, a.uten, a.vten, a.qrten, a.qsten, a.evapc, a.cufrc, a.qcu, a.qlu, a.qiu,
-                                   a.qc};
-        for (int q = 0; q < ADF_TR; ++q)
-            if (p == f[q]) return q;
-        if (p == a.precip) return ADF_TR + ncnst + ADC_PRECIP;
-        if (p == a.snow) return ADF_TR + ncnst + ADC_SNOW;
-        if (p == a.cbmf) return ADF_TR + ncnst + ADC_CBMF;
-        if (p == a.rliq) return ADF_TR + ncnst + ADC_RLIQ;
-        if (p == a.cnt) return ADF_TR + ncnst + ADC_CNT;
-        if (p == a.cnb) return ADF_TR + ncnst + ADC_CNB;
-        return ADF_TR + ncnst + ADC_CUSH;
-    }
     UWSHCU_HD inline D in(const double* p, int k) const {
         UW_CHECK(k <= mkx && k >= (iface(p) ? 0 : 1) && i >= 0 && i < a.ncol);
-        if constexpr (kAD) {
-            const int base = p == a.t0 ? ADI_T0 : p == a.qv0 ? ADI_QV0 : p == a.u0 ? ADI_U0 : p == a.v0 ? ADI_V0
-                           : p == a.tke ? ADI_TKE : -1;
-            if (base >= 0) return D(p[row(k)], base * KS + k);
-        }
         return D(p[row(k)]);
+    }
+    template <int F>
+    UWSHCU_HD inline D in(AdIn<F> p, int k) const {
+        UW_CHECK(k <= mkx && k >= (iface(p) ? 0 : 1) && i >= 0 && i < a.ncol);
+        if constexpr (kAD) return D(p[row(k)], F * KS + k);
+        else return p[row(k)];
     }
     // t0 and qv0 of layer k as the column physics sees them.  The modified scheme's
     // wrapper (zwshcu.F90:547-566) adds tpert / qpert, capped, to t0 / qv0 in every
@@ -326,14 +370,16 @@ struct Column {
         }
         return v;
     }
-    UWSHCU_HD inline D& out(double* p, int k) const {
+    template <int F>
+    UWSHCU_HD inline D& out(AdOut<F> p, int k) const {
         UW_CHECK(k <= mkx && k >= (iface(p) ? 0 : 1) && i >= 0 && i < a.ncol);
-        if constexpr (kAD) return adout(ad_field(p), k);
+        if constexpr (kAD) return adout(F, k);
         else return p[row(k)];
     }
     // column scalars (precip, snow, cbmf, rliq, cnt, cnb, cush)
-    UWSHCU_HD inline D& cout(double* p) const {
-        if constexpr (kAD) return adout(ad_field(p), 0);
+    template <int F>
+    UWSHCU_HD inline D& cout(AdScalar<F> p) const {
+        if constexpr (kAD) return adout(ADF_TR + ncnst + F, 0);
         else return p[i];
     }
     UWSHCU_HD inline D trin(int m, int k) const {   // m 1-based
@@ -360,7 +406,13 @@ struct Column {
         UW_CHECK(arr >= 0 && arr < ENV_ARRAYS && k >= 0 && k <= mkx && iw >= 0 && (long long)iw < (long long)wld);
         return env[((size_t)arr * KS + k) * wld + iw];
     }
-    UWSHCU_HD inline R Er(int arr, int k) const { return R(E(arr, k)); }
+    // A value of the environment as an operand; the Exner functions, of the pressures alone, are
+    // constants to the adjoint.
+    UWSHCU_HD inline D Ec(int arr, int k) const { return D(val(E(arr, k))); }
+    UWSHCU_HD inline R Er(int arr, int k) const {
+        if (kAD && (arr == A_EXN0 || arr == A_EXNS0)) return R(Ec(arr, k));
+        return R(E(arr, k));
+    }
     UWSHCU_HD inline R& W(int arr, int k) const {
         UW_CHECK(arr >= 0 && arr < WS_FIXED && k >= 0 && k <= mkx && iw >= 0 && (long long)iw < (long long)wld);
         return ws[((size_t)arr * KS + k) * wld + iw]; }
@@ -417,12 +469,12 @@ struct Column {
             const D pb = in(a.ps0, k - 1), pt = in(a.ps0, k), pm = in(a.p0, k);
             const D thl0bot = E(thl, k) + E(ssthl, k) * (pb - pm);
             const D qt0bot = E(qt, k) + E(ssqt, k) * (pb - pm);
-            if (T.conden_x(pb, E(A_EXNS0, k - 1), thl0bot, qt0bot, th, qv, ql, qi)) return false;
+            if (T.conden_x(pb, Ec(A_EXNS0, k - 1), thl0bot, qt0bot, th, qv, ql, qi)) return false;
             E(thvb, k) = th * (1.0 + C.zvir * qv - ql - qi);
             E(thvlb, k) = thl0bot * (1.0 + C.zvir * qt0bot);
             const D thl0top = E(thl, k) + E(ssthl, k) * (pt - pm);
             const D qt0top = E(qt, k) + E(ssqt, k) * (pt - pm);
-            if (T.conden_x(pt, E(A_EXNS0, k), thl0top, qt0top, th, qv, ql, qi)) return false;
+            if (T.conden_x(pt, Ec(A_EXNS0, k), thl0top, qt0top, th, qv, ql, qi)) return false;
             E(thvt, k) = th * (1.0 + C.zvir * qv - ql - qi);
             E(thvlt, k) = thl0top * (1.0 + C.zvir * qt0top);
         }
@@ -446,11 +498,11 @@ struct Column {
     }
     UWSHCU_HD UW_INLINE void env_mid_values(int k, D& thv0j, D& qs0) const {
         D th, qv, ql, qi, es;
-        if (T.conden_x(in(a.p0, k), E(A_EXN0, k), E(A_THL0, k), E(A_QT0, k), th, qv, ql, qi)) {
+        if (T.conden_x(in(a.p0, k), Ec(A_EXN0, k), E(A_THL0, k), E(A_QT0, k), th, qv, ql, qi)) {
             thv0j = -1.0;
         } else {
             thv0j = th * (1.0 + C.zvir * qv - ql - qi);
-            T.qsat_es_qs(E(A_THL0, k) * E(A_EXN0, k), in(a.p0, k), es, qs0);
+            T.qsat_es_qs(E(A_THL0, k) * Ec(A_EXN0, k), in(a.p0, k), es, qs0);
         }
     }
     // the launch keeps the environment's records: it reads the layer-mean saturation there
@@ -651,7 +703,7 @@ struct Column {
         const D qv0 = in_qv0(k), ql0 = in(a.ql0, k), qi0 = in(a.qi0, k), t0 = in_t0(k);
         const D qt0 = (qv0 + ql0 + qi0);
         E(A_QT0, k) = qt0;
-        E(A_THL0, k) = (t0 - C.xlv * ql0 / C.cp - C.xls * qi0 / C.cp) / E(A_EXN0, k);
+        E(A_THL0, k) = (t0 - C.xlv * ql0 / C.cp - C.xls * qi0 / C.cp) / Ec(A_EXN0, k);
     }
     // Returns the level's record (EnvLevelOf; the caller keeps it or not).
     UWSHCU_HD EnvLevelOf<D> setup_level2(int k) const {
@@ -678,9 +730,9 @@ struct Column {
         D thv0j, qs0 = 0.0;
         if (keeps_records()) env_mid_values(k, thv0j, qs0);
         else env_mid(k, thv0j, qs0);
-        return EnvLevelOf<D>{in(a.p0, k), in(a.dp0, k), E(A_EXN0, k), E(A_THV0BOT, k), E(A_THL0, k), E(A_QT0, k),
+        return EnvLevelOf<D>{in(a.p0, k), in(a.dp0, k), Ec(A_EXN0, k), E(A_THV0BOT, k), E(A_THL0, k), E(A_QT0, k),
                              in(a.u0, k), in(a.v0, k), thv0j, qs0, in(a.z0, k), E(A_THV0TOP, k), E(A_SSTHL0, k),
-                             E(A_SSQT0, k), E(A_SSU0, k), E(A_SSV0, k), in(a.ps0, k), E(A_EXNS0, k)};
+                             E(A_SSQT0, k), E(A_SSU0, k), E(A_SSV0, k), in(a.ps0, k), Ec(A_EXNS0, k)};
     }
 
     // S22 of a column's first pass, level-parallel (uwshcu.F90:4169-4329), after the
@@ -696,7 +748,7 @@ struct Column {
         const D t0s = in_t0(k) + out(a.sten, k) * a.dt / C.cp;
         const D qt0 = (qv0s + ql0s + qi0s);
         E(B_QT0, k) = qt0;
-        E(B_THL0, k) = (t0s - C.xlv * ql0s / C.cp - C.xls * qi0s / C.cp) / E(A_EXN0, k);
+        E(B_THL0, k) = (t0s - C.xlv * ql0s / C.cp - C.xls * qi0s / C.cp) / Ec(A_EXN0, k);
     }
     UWSHCU_HD void setup_level_b2(int k) const {
         const int j = k < mkx ? k : mkx - 1;
@@ -796,7 +848,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         const D qv0 = in_qv0(k), ql0 = in(a.ql0, k), qi0 = in(a.qi0, k), t0 = in_t0(k);
         const D qt0 = (qv0 + ql0 + qi0);
         E(A_QT0, k) = qt0;
-        E(A_THL0, k) = (t0 - C.xlv * ql0 / C.cp - C.xls * qi0 / C.cp) / E(A_EXN0, k);
+        E(A_THL0, k) = (t0 - C.xlv * ql0 / C.cp - C.xls * qi0 / C.cp) / Ec(A_EXN0, k);
     }
     slope([&](int k) { return E(A_THL0, k); }, A_SSTHL0);
     slope([&](int k) { return E(A_QT0, k); }, A_SSQT0);
@@ -957,13 +1009,13 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                     cinlcl = fmax(cin, 0.0);
                     cin = cinlcl;
                     thvubot = thvlsrc;
-                    if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                    if (T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                     thvutop = th * (1.0 + C.zvir * qvj - qlj - qij);
                     T.getbuoy(plcl, thv0lcl, in(a.ps0, k), E(e_thvt, k), thvubot, thvutop, plfc, cin);
                     if (plfc > 0.0) { klfc = k; break; }
                 } else {
                     thvubot = thvutop;
-                    if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                    if (T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                     thvutop = th * (1.0 + C.zvir * qvj - qlj - qij);
                     T.getbuoy(in(a.ps0, k - 1), E(e_thvb, k), in(a.ps0, k), E(e_thvt, k), thvubot, thvutop, plfc, cin);
                     if (plfc > 0.0) { klfc = k; break; }
@@ -972,9 +1024,9 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
         } else {
             cinlcl = 0.0;
             for (int k = kinv; k <= mkx - 1; ++k) {
-                if (T.conden_x(in(a.ps0, k - 1), E(A_EXNS0, k - 1), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                if (T.conden_x(in(a.ps0, k - 1), Ec(A_EXNS0, k - 1), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                 const D thvubot = th * (1.0 + C.zvir * qvj - qlj - qij);
-                if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                if (T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), thlsrc, qtsrc, th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                 const D thvutop = th * (1.0 + C.zvir * qvj - qlj - qij);
                 T.getbuoy(in(a.ps0, k - 1), E(e_thvb, k), in(a.ps0, k), E(e_thvt, k), thvubot, thvutop, plfc, cin);
                 if (plfc > 0.0) { klfc = k; break; }
@@ -1036,7 +1088,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             D sigmaw = sqrt(1.0 * tkeavg + 5.e-4);
             D rho0inv = 0.0;
             if constexpr (ZW) {
-                rho0inv = in(a.ps0, kinv - 1) / (C.r * E(A_THV0TOP, kinv - 1) * E(A_EXNS0, kinv - 1));
+                rho0inv = in(a.ps0, kinv - 1) / (C.r * E(A_THV0TOP, kinv - 1) * Ec(A_EXNS0, kinv - 1));
                 if (a.zw.pertw) {
                     // zwshcu.F90:2282-2285: a warm perturbation widens the w' distribution
                     const double tp = fmin(a.tpert[i], a.zw.tpertmax);
@@ -1055,7 +1107,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
             D mu = wcrit / sigmaw / 1.4142;
             if (mu >= 3.0) { exit_code = EX_MU3; goto L333; }
             if constexpr (!ZW)
-                rho0inv = in(a.ps0, kinv - 1) / (C.r * E(A_THV0TOP, kinv - 1) * E(A_EXNS0, kinv - 1));
+                rho0inv = in(a.ps0, kinv - 1) / (C.r * E(A_THV0TOP, kinv - 1) * Ec(A_EXNS0, kinv - 1));
             D cbmf_d = (rho0inv * sigmaw / 2.5066) * uexp(-(mu * mu));
             const D cbmflimit = 0.9 * in(a.dp0, kinv - 1) / C.g / dtd;
             D mumin0 = 0.0;
@@ -1345,7 +1397,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 }
                 const R thl_prog = Er(A_THL0, k) + thlten_sub * dt;
                 const R qt_prog = fmax(Er(A_QT0, k) + qtten_sub * dt, R(1.e-12));
-                if (T.conden_x(in(a.p0, k), E(A_EXN0, k), thl_prog, qt_prog, th, qvj, qlj, qij)) { exit_code = EX_SUBCONDEN; goto L333; }
+                if (T.conden_x(in(a.p0, k), Ec(A_EXN0, k), thl_prog, qt_prog, th, qvj, qlj, qij)) { exit_code = EX_SUBCONDEN; goto L333; }
                 W(W_QLSINK, k) = fmax(qlten_sub, -R(in(a.ql0, k)) / dt);
                 W(W_QISINK, k) = fmax(qiten_sub, -R(in(a.qi0, k)) / dt);
                 W(W_NLSINK, k) = fmax(nlten_sub, -trz(ixl, k) / dt);
@@ -1407,7 +1459,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                     qiubelow = R(qij);
                     qlr_base = qlubelow;
                     qir_base = qiubelow;
-                    if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                    if (T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                     qlr = R(qlj); qir = R(qij);
                     const R fr = (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
                     qlu_mid = R(0.5) * (qlubelow + qlr) * (prel - R(in(a.ps0, k))) / R(in(a.ps0, k - 1) - in(a.ps0, k));
@@ -1419,7 +1471,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                     qlu_mid = R(0.5) * (qlubelow + qlr) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
                     qiu_mid = R(0.5) * (qiubelow + qir) * (-ppen) / R(in(a.ps0, k - 1) - in(a.ps0, k));
                 } else {
-                    if (T.conden_x(in(a.ps0, k), E(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
+                    if (T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), W(W_THLU, k), W(W_QTU, k), th, qvj, qlj, qij)) { exit_code = EX_CONDEN; goto L333; }
                     qlr = R(qlj); qir = R(qij);
                     qlu_mid = R(0.5) * (qlubelow + qlr);
                     qiu_mid = R(0.5) * (qiubelow + qir);
@@ -1452,7 +1504,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                     nc_lm = nc_lm - g * umf_k * trz(ixl, k) / dps;
                     nc_im = nc_im - g * umf_k * trz(ixi, k) / dps;
                     D ql_e, qi_e;
-                    if (T.conden_x(in(a.p0, k), E(A_EXN0, k), W(W_THLUE, k), W(W_QTUE, k), th, qvj, ql_e, qi_e)) { exit_code = EX_KBUPCONDEN; goto L333; }
+                    if (T.conden_x(in(a.p0, k), Ec(A_EXN0, k), W(W_THLUE, k), W(W_QTUE, k), th, qvj, ql_e, qi_e)) { exit_code = EX_KBUPCONDEN; goto L333; }
                     const R nl_e = (ql_e > 0.0 && has_nl) ? WT(2, ixl, k) : R(0);
                     const R ni_e = (qi_e > 0.0 && has_ni) ? WT(2, ixi, k) : R(0);
                     const R emfk = W(W_EMF, k);
@@ -1629,7 +1681,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::run_body()
                 const D t0s = in_t0(k) + out(a.sten, k) * dtd / C.cp;
                 const D qt0 = (qv0s + ql0s + qi0s);
                 E(B_QT0, k) = qt0;
-                E(B_THL0, k) = (t0s - C.xlv * ql0s / C.cp - C.xls * qi0s / C.cp) / E(A_EXN0, k);
+                E(B_THL0, k) = (t0s - C.xlv * ql0s / C.cp - C.xls * qi0s / C.cp) / Ec(A_EXN0, k);
             }
             slope([&](int k) { return E(B_THL0, k); }, B_SSTHL0);
             slope([&](int k) { return E(B_QT0, k); }, B_SSQT0);

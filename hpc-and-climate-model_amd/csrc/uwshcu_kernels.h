@@ -30,6 +30,9 @@ hipError_t launch_check_columns(const FwdArgs& args, const uwshcu_consts* dconst
 // (args.ad holds the AD output values and the tape headers).  Sweep: zero adj[0, nadj)
 // (nadj = the pool's adj_next after the recording), then sweep each recorded tape from
 // the cotangents to the gradients.
+// Columns per wavefront of the adjoint's kernels: few enough that a launch has a wavefront
+// for each of the 1024 SIMDs where its columns allow.
+inline int adjoint_lanes(int n) { return n <= 8 * 1024 ? 8 : n <= 16 * 1024 ? 16 : n <= 32 * 1024 ? 32 : 64; }
 hipError_t launch_adjoint_record(const FwdArgs& args, int n, const uwshcu_consts* dconsts, const double* destbl,
                                  TapePool* pool, int* pages, int maxp, int cap, int* node_out, hipStream_t stream);
 hipError_t launch_adjoint_sweep(const FwdArgs& args, int n, double* adj, long long nadj, const int* node_out,

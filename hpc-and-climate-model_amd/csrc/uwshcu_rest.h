@@ -244,11 +244,11 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                     tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
                 W(W_QLR, krel - 1) = R(qlj);
                 W(W_QIR, krel - 1) = R(qij);
-                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
+                bad = T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
             } else if (k == kpen) {
                 bad = T.conden(R(in(a.ps0, k - 1)) + ppen, thlu_top, qtu_top, th, qvj, qlj, qij);
             } else {
-                bad = T.conden_x(in(a.ps0, k), E(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
+                bad = T.conden_x(in(a.ps0, k), Ec(A_EXNS0, k), P(W_THLU, k), P(W_QTU, k), th, qvj, qlj, qij);
             }
             if (bad) tm.fail((1 << 16) | (k << 4) | EX_CONDEN);
             W(W_QLR, k) = R(qlj);
@@ -367,7 +367,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
             }
             const R thl_prog = thl0k + thlten_sub * dt;
             const R qt_prog = fmax(qt0k + qtten_sub * dt, R(1.e-12));
-            if (T.conden_x(in(a.p0, k), E(A_EXN0, k), thl_prog, qt_prog, th, qvj, qlj, qij))
+            if (T.conden_x(in(a.p0, k), Ec(A_EXN0, k), thl_prog, qt_prog, th, qvj, qlj, qij))
                 tm.fail((k << 4) | EX_SUBCONDEN);
             const R qlsink = fmax(qlten_sub, -ql0k / dt), qisink = fmax(qiten_sub, -qi0k / dt);
             const R nlsink = fmax(nlten_sub, -trz(ixl, k) / dt), nisink = fmax(niten_sub, -trz(ixi, k) / dt);
@@ -440,7 +440,7 @@ UWSHCU_HD __attribute__((always_inline)) void Column<R, D, ZW, FAST>::rest_team(
                 nc_lm = nc_lm - g * umf_k * trz(ixl, k) / dps;
                 nc_im = nc_im - g * umf_k * trz(ixi, k) / dps;
                 D ql_e, qi_e;
-                if (T.conden_x(in(a.p0, k), E(A_EXN0, k), W(W_THLUE, k), W(W_QTUE, k), th, qvj, ql_e, qi_e))
+                if (T.conden_x(in(a.p0, k), Ec(A_EXN0, k), W(W_THLUE, k), W(W_QTUE, k), th, qvj, ql_e, qi_e))
                     tm.fail((1 << 16) | (k << 4) | EX_KBUPCONDEN);
                 const R nl_e = (ql_e > 0.0 && has_nl) ? WT(2, ixl, k) : R(0);
                 const R ni_e = (qi_e > 0.0 && has_ni) ? WT(2, ixi, k) : R(0);

@@ -21,7 +21,7 @@ UWSHCU_HD UW_INLINE EnvLevelOf<D> Column<R, D, ZW, FAST>::env_level_lower(int k)
         e.p0 = p.x; e.dp0 = p.y; e.exn0 = q.x; e.thv0bot = q.y; e.thl0 = s.x; e.qt0 = s.y; e.u0 = t.x; e.v0 = t.y;
         return e;
     }
-    e.p0 = in(a.p0, k); e.dp0 = in(a.dp0, k); e.exn0 = E(A_EXN0, k); e.thv0bot = E(A_THV0BOT, k);
+    e.p0 = in(a.p0, k); e.dp0 = in(a.dp0, k); e.exn0 = Ec(A_EXN0, k); e.thv0bot = E(A_THV0BOT, k);
     e.thl0 = E(A_THL0, k); e.qt0 = E(A_QT0, k); e.u0 = in(a.u0, k); e.v0 = in(a.v0, k);
     return e;
 }
@@ -36,7 +36,7 @@ UWSHCU_HD UW_INLINE EnvLevelOf<D> Column<R, D, ZW, FAST>::env_level_upper(int k)
         return e;
     }
     e.z0 = in(a.z0, k); e.thv0top = E(A_THV0TOP, k); e.ssthl = E(A_SSTHL0, k); e.ssqt = E(A_SSQT0, k);
-    e.ssu = E(A_SSU0, k); e.ssv = E(A_SSV0, k); e.ps0 = in(a.ps0, k); e.exns0 = E(A_EXNS0, k);
+    e.ssu = E(A_SSU0, k); e.ssv = E(A_SSV0, k); e.ps0 = in(a.ps0, k); e.exns0 = Ec(A_EXNS0, k);
     return e;
 }
 template <class R, class D, bool ZW, bool FAST>

@@ -226,17 +226,17 @@ hipError_t launch_adjoint_sweep(const FwdArgs& args, int n, double* adj, long lo
         if (blocks > 8192) blocks = 8192;
         hipLaunchKernelGGL(zero_kernel, dim3((unsigned)blocks), dim3(256), 0, stream, adj, nadj);
     }
-    // Columns per wavefront: few enough that a launch has a wavefront for every SIMD (1024)
-    // where its columns allow.
     auto sweep = [&](auto kernel, int lanes) {
         hipLaunchKernelGGL(kernel, dim3((n + lanes - 1) / lanes), dim3(64), 0, stream, n, args.col0, args.mkx,
                            args.ncnst, args.wld, (long long)args.ldc, (const TapeCtx*)args.ad.tapes, node_out, adj, cot,
                            g);
     };
-    if (n <= 8 * 1024) sweep(adjoint_sweep_kernel<8>, 8);
-    else if (n <= 16 * 1024) sweep(adjoint_sweep_kernel<16>, 16);
-    else if (n <= 32 * 1024) sweep(adjoint_sweep_kernel<32>, 32);
-    else sweep(adjoint_sweep_kernel<64>, 64);
+    switch (adjoint_lanes(n)) {
+    case 8: sweep(adjoint_sweep_kernel<8>, 8); break;
+    case 16: sweep(adjoint_sweep_kernel<16>, 16); break;
+    case 32: sweep(adjoint_sweep_kernel<32>, 32); break;
+    default: sweep(adjoint_sweep_kernel<64>, 64);
+    }
     return hipGetLastError();
 }
 
