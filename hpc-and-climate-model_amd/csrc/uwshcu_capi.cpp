@@ -20,6 +20,14 @@
 
 using uwshcu::FwdArgs;
 
+// The host-pointer entry points copy through a ring of pinned slots, which the host fills or
+// empties while others move: an asynchronous copy from or to ordinary memory
+// cost 0.13 ms whatever its size, and a chunk has 45 arrays (a call of 512 x 30 x 5 took 7.9 ms,
+// with the ring 2.4; of 65536 x 35 x 3 47 and 34).  A ring, not the chunk's size: pinning
+// takes 0.4 ms per MiB of a context's first call.
+constexpr int kHostSlots = 8;
+constexpr size_t kHostSlotBytes = (size_t)1 << 20;
+
 struct uwshcu_ctx {
     int device = 0;
     uwshcu_consts consts{};
@@ -35,6 +43,8 @@ struct uwshcu_ctx {
     size_t stage_bytes = 0;
     int* d_diag = nullptr;
     size_t diag_bytes = 0;
+    char* h_ring = nullptr;      // HostRing's pinned memory and events
+    hipEvent_t h_ring_event[kHostSlots] = {};
     // mixed precision: input cush copy, branch flags, recompute list and its length
     double* d_cush_in = nullptr;
     int* d_amb = nullptr;
@@ -685,6 +695,9 @@ int uwshcu_ctx_destroy(uwshcu_ctx* ctx) {
     if (ctx->d_defer) (void)hipFree(ctx->d_defer);
     if (ctx->d_defer_state) (void)hipFree(ctx->d_defer_state);
     if (ctx->d_rec) (void)hipFree(ctx->d_rec);
+    if (ctx->h_ring) (void)hipHostFree(ctx->h_ring);
+    for (hipEvent_t e : ctx->h_ring_event)
+        if (e) (void)hipEventDestroy(e);
     if (ctx->d_packed) (void)hipFree(ctx->d_packed);
     if (ctx->d_ctab) (void)hipFree(ctx->d_ctab);
     if (ctx->h_ctab) (void)hipHostFree(ctx->h_ctab);
@@ -1015,6 +1028,105 @@ int uwshcu_status(uwshcu_ctx* ctx, void* stream, int* bad_col) {
     return h[0];
 }
 
+namespace {
+
+// Copies between host arrays and device staging through a context's pinned slots, on one
+// stream.  put() may be followed by more of the same region (ship() sends the rest); get()
+// returns when its arrays are filled.  After a failure nothing more is copied.
+struct HostRing {
+    struct Rows {       // a host array of rows of `pitch` bytes, of which `width` are copied
+        void* host;
+        size_t rows;
+    };
+    uwshcu_ctx* ctx;
+    hipStream_t st;
+    bool ok = true;
+    bool busy[kHostSlots] = {};
+    int slot = 0;
+    size_t fill = 0;
+    char* dev = nullptr;    // where the slot being filled goes
+
+    int open() {
+        if (!ctx->h_ring &&
+            !hip_ok(hipHostMalloc((void**)&ctx->h_ring, kHostSlots * kHostSlotBytes, hipHostMallocDefault))) {
+            ctx->h_ring = nullptr;
+            return UWSHCU_ERR_NOMEM;
+        }
+        for (hipEvent_t& e : ctx->h_ring_event)
+            if (!e && !hip_ok(hipEventCreateWithFlags(&e, hipEventDisableTiming))) return UWSHCU_ERR_HIP;
+        return UWSHCU_OK;
+    }
+    char* mem(int s) { return ctx->h_ring + (size_t)s * kHostSlotBytes; }
+    void wait(int s) {      // until slot s's copy is done
+        if (busy[s]) ok = hip_ok(hipEventSynchronize(ctx->h_ring_event[s])) && ok;
+        busy[s] = false;
+    }
+    void copy(int s, void* to, const void* from, size_t n, hipMemcpyKind kind) {
+        if (!ok) return;
+        ok = hip_ok(hipMemcpyAsync(to, from, n, kind, st)) && hip_ok(hipEventRecord(ctx->h_ring_event[s], st));
+        busy[s] = true;
+    }
+    void put(void* to, const void* from, size_t n) {
+        const char* h = static_cast<const char*>(from);
+        if (fill == 0) dev = static_cast<char*>(to);
+        while (n && ok) {
+            if (fill == 0) wait(slot);
+            const size_t m = n < kHostSlotBytes - fill ? n : kHostSlotBytes - fill;
+            std::memcpy(mem(slot) + fill, h, m);
+            fill += m;
+            h += m;
+            n -= m;
+            if (fill == kHostSlotBytes) ship();
+        }
+    }
+    void ship() {
+        if (fill) copy(slot, dev, mem(slot), fill, hipMemcpyHostToDevice);
+        dev += fill;
+        fill = 0;
+        slot = (slot + 1) % kHostSlots;
+    }
+    // The arrays that follow each other from device address `from` on.
+    void get(const void* from, const Rows* a, int na, size_t pitch, size_t width) {
+        size_t total = 0;
+        for (int q = 0; q < na; ++q) total += a[q].rows * pitch;
+        const char* d = static_cast<const char*>(from);
+        const size_t pieces = (total + kHostSlotBytes - 1) / kHostSlotBytes;
+        auto size = [&](size_t p) { return p + 1 < pieces ? kHostSlotBytes : total - p * kHostSlotBytes; };
+        auto issue = [&](size_t p) {
+            copy((int)(p % kHostSlots), mem((int)(p % kHostSlots)), d + p * kHostSlotBytes, size(p), hipMemcpyDeviceToHost);
+        };
+        for (size_t p = 0; p < pieces && p < (size_t)kHostSlots; ++p) issue(p);
+        int q = 0;
+        size_t a0 = 0;      // byte where array q begins
+        for (size_t p = 0; p < pieces && ok; ++p) {
+            const int s = (int)(p % kHostSlots);
+            wait(s);
+            const size_t b = p * kHostSlotBytes, e = b + size(p);
+            while (ok && q < na) {
+                const size_t a1 = a0 + a[q].rows * pitch;
+                const size_t lo = a0 > b ? a0 : b, hi = a1 < e ? a1 : e;
+                char* const host = static_cast<char*>(a[q].host);
+                if (width == pitch) {
+                    if (hi > lo) std::memcpy(host + (lo - a0), mem(s) + (lo - b), hi - lo);
+                } else {
+                    for (size_t x = lo; x < hi;) {     // row by row: x within a row, its copied part ends at w
+                        const size_t row = a0 + (x - a0) / pitch * pitch, w = row + width < hi ? row + width : hi;
+                        if (w > x) std::memcpy(host + (x - a0), mem(s) + (x - b), w - x);
+                        x = row + pitch;
+                    }
+                }
+                if (a1 > e) break;
+                a0 = a1;
+                ++q;
+            }
+            if (ok && p + kHostSlots < pieces) issue(p + kHostSlots);
+        }
+        if (!ok) (void)hipStreamSynchronize(st);
+    }
+};
+
+}  // namespace
+
 // Host-array forward: stage the inputs to the device, run, copy the outputs back.
 // zwp != nullptr selects the modified scheme, whose host inputs omega_h (pcols, pver)
 // and tpert_h, qpert_h (pcols) are staged too.
@@ -1063,14 +1175,15 @@ static int forward_host_impl(uwshcu_ctx* ctx, int precision, const uwshcu_params
         }
         ddiag = ctx->d_diag;
     }
+    hipStream_t st = ctx->stream;
+    HostRing ring{ctx, st};
+    if (int e = ring.open()) return e;
     double* base = ctx->d_stage;
     size_t off = 0;
     auto take = [&](size_t n) { double* p = base + off; off += n; return p; };
-    hipStream_t st = ctx->stream;
-    bool ok = true;
     auto h2d = [&](const double* h, size_t n) {
         double* d = take(n);
-        if (n) ok = ok && hip_ok(hipMemcpyAsync(d, h, n * sizeof(double), hipMemcpyHostToDevice, st));
+        ring.put(d, h, n * sizeof(double));
         return (const double*)d;
     };
     Chunk ch{};
@@ -1080,13 +1193,14 @@ static int forward_host_impl(uwshcu_ctx* ctx, int precision, const uwshcu_params
     ch.t0 = h2d(t0, L); ch.s0 = h2d(s0, L);
     ch.tr0 = h2d(tr0, T);
     ch.pblh = h2d(pblh, S);
-    ch.cush = const_cast<double*>(h2d(cush, S));
     ZwInputs zin{zwp, nullptr, nullptr, nullptr};
     if (zwp) {
         zin.omega = h2d(omega_h, L);
         zin.tpert = h2d(tpert_h, S);
         zin.qpert = h2d(qpert_h, S);
     }
+    ch.cush = const_cast<double*>(h2d(cush, S));   // the last input, in front of the outputs: it is one of them
+    ring.ship();
     ch.umf = take(I); ch.slflx = take(I); ch.qtflx = take(I); ch.flxprc1 = take(I); ch.flxsnow1 = take(I);
     ch.wu = take(I);
     ch.qvten = take(L); ch.qlten = take(L); ch.qiten = take(L); ch.sten = take(L); ch.uten = take(L);
@@ -1094,34 +1208,30 @@ static int forward_host_impl(uwshcu_ctx* ctx, int precision, const uwshcu_params
     ch.qcu = take(L); ch.qlu = take(L); ch.qiu = take(L); ch.qc = take(L);
     ch.trten = take(T);
     ch.precip = take(S); ch.snow = take(S); ch.cbmf = take(S); ch.rliq = take(S); ch.cnt = take(S); ch.cnb = take(S);
-    if (!ok) return UWSHCU_ERR_HIP;
-    int rc = run_device(ctx, precision, par, pcols, ncol, pver, ncnst, dt, ch, ddiag, st, zwp ? &zin : nullptr);
-    if (rc) return rc;
+    int rc = ring.ok ? run_device(ctx, precision, par, pcols, ncol, pver, ncnst, dt, ch, ddiag, st, zwp ? &zin : nullptr)
+                     : UWSHCU_ERR_HIP;
+    if (rc) {
+        (void)hipStreamSynchronize(st);   // the slots are the next call's
+        return rc;
+    }
     // outputs: the first ncol columns of each row only (the caller's padding columns
     // ncol..pcols-1 stay as they were, as in the reference, which writes 1:iend)
     const size_t rows_i = (size_t)pver + 1, rows_l = (size_t)pver, rows_t = (size_t)pver * ncnst;
-    auto d2h = [&](void* h, const void* d, size_t rows, size_t elem) {
-        if (rows)
-            ok = ok && hip_ok(hipMemcpy2DAsync(h, (size_t)pcols * elem, d, (size_t)pcols * elem, (size_t)ncol * elem,
-                                               rows, hipMemcpyDeviceToHost, st));
-    };
-    const size_t e8 = sizeof(double);
-    d2h(cush, ch.cush, 1, e8);
-    d2h(umf, ch.umf, rows_i, e8); d2h(slflx, ch.slflx, rows_i, e8); d2h(qtflx, ch.qtflx, rows_i, e8);
-    d2h(flxprc1, ch.flxprc1, rows_i, e8); d2h(flxsnow1, ch.flxsnow1, rows_i, e8); d2h(wu, ch.wu, rows_i, e8);
-    d2h(qvten, ch.qvten, rows_l, e8); d2h(qlten, ch.qlten, rows_l, e8); d2h(qiten, ch.qiten, rows_l, e8);
-    d2h(sten, ch.sten, rows_l, e8); d2h(uten, ch.uten, rows_l, e8); d2h(vten, ch.vten, rows_l, e8);
-    d2h(qrten, ch.qrten, rows_l, e8); d2h(qsten, ch.qsten, rows_l, e8); d2h(evapc, ch.evapc, rows_l, e8);
-    d2h(cufrc, ch.cufrc, rows_l, e8); d2h(qcu, ch.qcu, rows_l, e8); d2h(qlu, ch.qlu, rows_l, e8);
-    d2h(qiu, ch.qiu, rows_l, e8); d2h(qc, ch.qc, rows_l, e8);
-    d2h(trten, ch.trten, rows_t, e8);
-    d2h(precip, ch.precip, 1, e8); d2h(snow, ch.snow, 1, e8); d2h(cbmf, ch.cbmf, 1, e8); d2h(rliq, ch.rliq, 1, e8);
-    d2h(cnt, ch.cnt, 1, e8); d2h(cnb, ch.cnb, 1, e8);
-    if (diag) d2h(diag, ddiag, UWSHCU_NDIAG, sizeof(int));
+    const HostRing::Rows outs[] = {   // in the order of their addresses
+        {cush, 1}, {umf, rows_i}, {slflx, rows_i}, {qtflx, rows_i}, {flxprc1, rows_i}, {flxsnow1, rows_i},
+        {wu, rows_i}, {qvten, rows_l}, {qlten, rows_l}, {qiten, rows_l}, {sten, rows_l}, {uten, rows_l},
+        {vten, rows_l}, {qrten, rows_l}, {qsten, rows_l}, {evapc, rows_l}, {cufrc, rows_l}, {qcu, rows_l},
+        {qlu, rows_l}, {qiu, rows_l}, {qc, rows_l}, {trten, rows_t}, {precip, 1}, {snow, 1}, {cbmf, 1},
+        {rliq, 1}, {cnt, 1}, {cnb, 1}};
+    ring.get(ch.cush, outs, (int)(sizeof(outs) / sizeof(outs[0])), pcols * sizeof(double), ncol * sizeof(double));
+    if (diag) {
+        const HostRing::Rows rows{diag, UWSHCU_NDIAG};
+        ring.get(ddiag, &rows, 1, pcols * sizeof(int), ncol * sizeof(int));
+    }
     int h[2] = {0, -1};
-    ok = ok && hip_ok(hipMemcpyAsync(h, ctx->d_err, sizeof(h), hipMemcpyDeviceToHost, st)) &&
-         hip_ok(hipStreamSynchronize(st)) && hip_ok(uwshcu::launch_clear_status(ctx->d_err, st));
-    if (!ok) return UWSHCU_ERR_HIP;
+    const HostRing::Rows err{h, 1};
+    ring.get(ctx->d_err, &err, 1, sizeof(h), sizeof(h));
+    if (!ring.ok || !hip_ok(uwshcu::launch_clear_status(ctx->d_err, st))) return UWSHCU_ERR_HIP;
     if (bad_col) *bad_col = h[0] ? h[1] : -1;
     return h[0];
 }
