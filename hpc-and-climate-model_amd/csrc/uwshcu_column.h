@@ -172,19 +172,19 @@ struct FwdArgs {
     const double* cush_in;   // optional: read the input cush here instead of from cush
     int* amb_flag;           // optional [ldc]: 1 where an FP32 branch decision was within rounding
     int env_ready;           // 1: setup_level1/2 already filled the set-A environment and the wet bulb
-    // optional: a column whose implicit-CIN pass needs a second convection pass stops
-    // there, saves its scalars (NRESUME doubles, [field][slot], wld apart) in
-    // defer_state, leaves its outputs to be rewritten and appends itself to defer_list
+    // The parts of a split launch: a column that reaches the cloud-base closure saves its
+    // scalars (NRESUME doubles, [field][slot], wld apart) in defer_state, leaves its outputs
+    // to be rewritten and marks its slot in defer_mark, from which the list of the next
+    // parts is made (or, without defer_mark, appends itself to defer_list).
     int* defer_list;
     int* defer_count;
     double* defer_state;
-    // optional: the environment of each level as one record (EnvLevelOf), slot by slot
+    // the environment of each level as one record (EnvLevelOf), slot by slot
     double* rec;
-    // 1 (with defer_list): a column that reaches the cloud-base closure of its first
-    // pass stops there instead, saves its scalars and lists itself, so that only the
-    // triggered columns run the convection stages, packed densely in a launch of their own
+    // 1 (with defer_list, columns run whole): it stops at its first pass's closure, else only
+    // before its second convection pass
     int defer_at_closure;
-    int* defer_mark;         // optional [wld]: mark the deferred column's slot 1 instead of listing it
+    int* defer_mark;         // [wld]
     // 1: continue each listed column at the closure of its first pass; 2: at its second
     // convection pass; 4: at the implicit-CIN iteration
     int resume;
@@ -247,7 +247,7 @@ enum { EX_NONE = 0, EX_CONDEN = 1, EX_KINV1 = 2, EX_KLCLMKX = 3, EX_KLFCMKX = 4,
 // of the arguments in scratch, reloads each array pointer from it, and, unable to tell
 // global from LDS memory behind those pointers, issues flat instructions.  Expanded,
 // the pointers stay in scalar registers and every access is a global or LDS one
-// (scratch 1.2 KB -> 44 B per lane in the one-wavefront build).
+// (scratch 1.2 KB -> 44 B per lane in a kernel of the whole column pass).
 #define UW_INLINE __attribute__((always_inline))
 
 // The environment of layer k, and of its top interface, as the buoyancy sorting reads it.
@@ -676,11 +676,10 @@ struct Column {
     template <int PART>
     UWSHCU_HD void run_part() const;
     // the column pass itself, expanded into each forward kernel so that each gets its
-    // own register allocation (the two builds differ in their register budget).
-    // kSplit = false leaves out what only the launches of a split large launch do (stop
-    // at, and continue from, the closure, the buoyancy sorting or the second pass),
-    // which the one-wavefront-per-SIMD build never runs.  PART (PART_*) fixes which part
-    // of a split launch runs.
+    // own register allocation.
+    // kSplit = false leaves out what only the parts of a split launch do (stop at, and
+    // continue from, the closure, the buoyancy sorting or the second pass), which the
+    // adjoint's recording never runs.  PART (PART_*) fixes which part runs.
     template <bool kSplit, int PART = PART_ALL>
     UWSHCU_HD __attribute__((always_inline)) void run_body() const;
 

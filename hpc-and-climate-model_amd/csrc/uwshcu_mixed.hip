@@ -3,7 +3,7 @@
 // cloud-base closure, environment, wet bulb and positive-moisture fix-up.  After the
 // FP32 pass, check_columns_kernel lists the columns that fail the FP64 conservation
 // check or took an FP32 branch decision within rounding; the driver recomputes
-// exactly those in FP64 (forward_kernel<double> over the list).
+// exactly those in FP64 (the FP64 pipeline over the list).
 #include "uwshcu_check.h"
 #include "uwshcu_forward.h"
 
