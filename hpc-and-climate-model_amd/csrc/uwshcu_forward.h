@@ -136,7 +136,7 @@ void sort_kernel(FwdArgs args, int n, int second_pass, int* queue, const uwshcu_
 
 // S12-S21 of the listed columns: a workgroup takes 64 of them, wavefront w the levels
 // w, w + kRestWaves, ... (uwshcu_rest.h).  Bound by memory: it waits for loads and stores of
-// 34 GB at 1 036 800 x 35 x 3.  Four wavefronts, two workgroups on a CU: both passes take
+// 40 GB at 1 036 800 x 35 x 3.  Four wavefronts, two workgroups on a CU: both passes take
 // 11.0 ms there, with eight 12.2; with four the stages that one wavefront runs
 // alone leave fewer idle.  The fast path's saturation adjustment takes more registers than
 // two workgroups leave; held to them (with spills) its two passes take 7.9 ms, else 9.5.

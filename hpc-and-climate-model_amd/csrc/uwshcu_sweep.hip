@@ -24,8 +24,8 @@ namespace uwshcu {
 //    in the window; the next batch's nodes are loaded before a batch's steps and their
 //    page-table entry a batch earlier still;
 //  - a step reads one window entry and adds to two without waiting (LDS FP64 adds).
-// 27.7 to 23.1 ms there; at 4097 x 72 x 10, where L = 8 gives 513 wavefronts instead of 65,
-// 58.6 to 35 ms.
+// 28.5 to 22.5 ms there; at 4097 x 72 x 10, where L = 8 gives 513 wavefronts instead of 65,
+// 57.6 to 36.4 ms.
 //
 // LDS: a window of 64 recent adjoints and its spare entry (520 B per column) and the four
 // nodes, 40 448 B at L = 64: four workgroups a CU, one wavefront per SIMD.
