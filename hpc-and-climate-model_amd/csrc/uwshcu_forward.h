@@ -64,7 +64,8 @@ void forward_kernel_part(FwdArgs args, int n, const uwshcu_consts* __restrict__ 
 // launch), so a wavefront's columns stay near each other in memory.  Lanes whose column
 // has reached its cloud top wait until kSortReady of them have (or none has a level left):
 // a cloud-top stage and a start cost a wavefront a quarter of a level, however few
-// lanes take them (waiting for 1, 6, 12 and 24 measured 13.4, 13.6, 13.8 and 13.6 ms without records).
+// lanes take them (waiting for 2, 6, 12 and 20 lanes: 9.4, 9.4, 9.6, 10.0 ms at 1036800 x 35 x 3
+// and 12.5, 11.5, 12.2, 13.1 at 200003 x 72 x 10).
 constexpr int kSortReady = 6;
 template <class R, bool ZW, bool FAST, int OCC>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(OCC)))
